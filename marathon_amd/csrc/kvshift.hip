@@ -356,7 +356,10 @@ struct ShiftParams {
   int32_t xcd_per;       // set at launch: tiles per XCD with xcds > 1, else 0
   int32_t layer_groups;  // the layer-major grid: 1 = asked for (host), then the layer
                          // groups at launch; 0: two-dimensional
-  int32_t pad3;
+  int32_t segs;          // workgroups per token (set_tiles); 1: a tile of whole tokens
+  uint32_t segs_magic;   // ceil(2^32 / segs): tile / segs == umulhi(tile, magic); 0: segs 1
+  int32_t sweep_rows;    // rows of a segment (segs > 1), or at least a tile's
+  uint32_t lane_magic;   // ceil(2^16 / chunks_per_row): lane / chunks_per_row
 };
 
 // A small shift's tables, carried in the launch's kernel arguments (no device copy):
@@ -950,7 +953,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
   const int wave = uniform(tid >> 6);
   const int nK = p.chunks_per_row;
   const int rpw = p.rows_per_wave;
-  const int row_in_wave = lane / nK;
+  const int row_in_wave = static_cast<int>((static_cast<uint32_t>(lane) * p.lane_magic) >> 16);
   const int j = lane - row_in_wave * nK;  // chunk index inside K (and inside V)
   const bool lane_live = row_in_wave < rpw;
   const int P = p.rotary / (2 * C);  // rotate_half distance, in chunks
@@ -969,7 +972,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
   } else if constexpr (!DIRECT) {
     asm volatile("" ::"s"(p.recs), "s"(p.src_k_base), "s"(p.src_v_base), "s"(p.dst_k_base),
                  "s"(p.dst_v_base), "s"(p.tables), "s"(p.k_scale), "s"(p.src_hstride),
-                 "s"(p.dst_hstride));
+                 "s"(p.dst_hstride), "s"(p.sweep_rows));
   } else if constexpr (!SMALL) {
     asm volatile("" ::"s"(p.starts), "s"(p.spans), "s"(p.n_spans));
   }
@@ -996,7 +999,13 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
     tile = static_cast<int64_t>(blockIdx.x % MKV_XCDS) * p.xcd_per + blockIdx.x / MKV_XCDS;
   }
   const int layer0 = lgroup * LB;
-  const int64_t g0 = tile * p.tile_tokens;
+  // a token of more rows than one sweep: its segments are workgroups of their own, one
+  // after the other in tile order (set_tiles).  No branch: behind one, the fields below
+  // would be fetched in one more dependent batch ahead of the data (3% of a 33 MB launch).
+  const uint32_t piece = static_cast<uint32_t>(tile);
+  const uint32_t whole = p.segs_magic != 0 ? __umulhi(piece, p.segs_magic) : piece;
+  const int seg_row = static_cast<int>(piece - whole * static_cast<uint32_t>(p.segs)) * p.sweep_rows;
+  const int64_t g0 = static_cast<int64_t>(whole) * p.tile_tokens;
   if constexpr (DIRECT && !SMALL) {
     // one workgroup checks the caller's prefix against the span table: starts[0] == 0,
     // each step equals the span's token count, and the last is at most total_tokens
@@ -1014,7 +1023,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
   const int64_t left = p.total_tokens - g0;
   if (left <= 0) return;  // padding workgroups of the XCD-aware grid
   const int ntok = static_cast<int>(left < p.tile_tokens ? left : p.tile_tokens);
-  const int nrows = ntok * H;
+  const int nrows = min(seg_row + p.sweep_rows, ntok * H);
   // small: the spans of the workgroup's tokens [g0, g0 + ntok), whose rotation tables the
   // workgroup computes together into LDS ([span - small_lo][2][rotary])
   float* small_tab = nullptr;
@@ -1167,7 +1176,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
       __syncthreads();
     }
   }
-  for (int r0 = 0; r0 < nrows; r0 += kWaves * U * rpw) {
+  for (int r0 = seg_row; r0 < nrows; r0 += kWaves * U * rpw) {
     // ---- phase A: where each pass reads and writes (uniform when UNIFORM).  All token
     // metadata is fetched first, then all base addresses, so the workgroup pays two
     // metadata round trips in total rather than two per pass; a token's metadata serves
@@ -1626,6 +1635,7 @@ struct Geometry {
   int chunks_per_row;
   int rows_per_wave;
   int tile_tokens;
+  int sweep_rows;  // rows one sweep of a workgroup covers
   bool uniform;
   uint32_t heads_magic;
   int xcds;  // the tile order (MKV_XCD_MIN_TOKEN_BYTES)
@@ -1654,6 +1664,7 @@ int check_geometry(int dtype, int heads, int head_size, int rotary, int64_t src_
   g.rows_per_wave = 64 / g.chunks_per_row;
   g.uniform = heads % g.rows_per_wave == 0;
   const int rows = g.rows_per_wave * kWaves * passes_of(dtype, g.uniform);
+  g.sweep_rows = rows;
   g.tile_tokens = rows / heads > 0 ? rows / heads : 1;
   // row -> (token, head) uses a 32-bit reciprocal, exact while rows < 2^16
   if (static_cast<int64_t>(g.tile_tokens) * heads >= (1 << 16))
@@ -1669,6 +1680,37 @@ int check_geometry(int dtype, int heads, int head_size, int rotary, int64_t src_
   if (src_hs < 0 || dst_hs < 0 || lane_max >= (int64_t{1} << 31))
     return fail(MKV_ERR_UNSUPPORTED, "head strides out of range");
   return MKV_OK;
+}
+
+// The tiles of a shift of `tokens` tokens, and how they map to rows (sp's tile fields).
+//
+// A token of more rows than one sweep of a workgroup (2-byte elements: more than 8 KV
+// heads of 128, or 4 of 256) is cut into segments of one sweep, each a workgroup of its
+// own: looping over them in one workgroup leaves its later loads queued behind its earlier
+// stores, and one launch per layer with too few waves to cover that.  Whole calls, one
+// workgroup a token against one a segment: a plan of 16 heads of 256, bf16, 28 layers,
+// 3,001 tokens 500 / 439 us (5.5 / 6.3 TB/s), 16 heads of 128, 40 layers, 4,096 tokens 438 / 420
+// us, 40 one-layer launches of the latter 605 / 529 us.  A segment's number comes from a 32-bit
+// reciprocal; where that would not be exact over the grid (billions of segments), a
+// workgroup keeps the whole token.
+int64_t set_tiles(const Geometry& g, int64_t tokens, ShiftParams& sp) {
+  sp.tile_tokens = g.tile_tokens;
+  sp.segs = 1;
+  sp.segs_magic = 0;
+  sp.sweep_rows = 1 << 16;  // a tile has fewer rows (check_geometry)
+  const int64_t segs = (sp.heads + g.sweep_rows - 1) / g.sweep_rows;
+  if (segs > 1 && tokens <= 0x7FFFFFFF / segs - MKV_XCDS) {
+    const uint64_t magic = ((uint64_t{1} << 32) + segs - 1) / segs;
+    const uint64_t excess = magic * segs - (uint64_t{1} << 32);
+    const uint64_t grid = static_cast<uint64_t>(tokens * segs) + MKV_XCDS;  // padded
+    if (grid * excess < (uint64_t{1} << 32)) {
+      sp.segs = static_cast<int32_t>(segs);
+      sp.segs_magic = static_cast<uint32_t>(magic);
+      sp.sweep_rows = g.sweep_rows;
+      return tokens * segs;
+    }
+  }
+  return (tokens + g.tile_tokens - 1) / g.tile_tokens;
 }
 
 template <int DT, bool BATCHED, bool UNIFORM, bool DIRECT, int LB>
@@ -1887,13 +1929,13 @@ extern "C" int mkv_scatter_shifted(const void* src, int64_t src_token_stride,
   sp.layers = 1;
   sp.heads = heads;
   sp.rotary = rot ? rotary : 0;
-  sp.tile_tokens = g.tile_tokens;
   sp.xcds = g.xcds;
   sp.chunks_per_row = g.chunks_per_row;
   sp.rows_per_wave = g.rows_per_wave;
+  sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
   sp.rotate = rot ? 1 : 0;
-  const int64_t tiles = (n_tokens + g.tile_tokens - 1) / g.tile_tokens;
+  const int64_t tiles = set_tiles(g, n_tokens, sp);
   return launch_any<false>(dtype, g.uniform, 0, sp, tiles, 1,
                            static_cast<hipStream_t>(stream));
 }
@@ -1927,8 +1969,8 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
     return fail(MKV_ERR_ARG, "token_order and order %d together: one order or the other",
                 d->order);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t tiles = (d->total_tokens + g.tile_tokens - 1) / g.tile_tokens;
-  if (tiles > 0x7FFFFFFF) return fail(MKV_ERR_UNSUPPORTED, "total_tokens too large");
+  if ((d->total_tokens + g.tile_tokens - 1) / g.tile_tokens > 0x7FFFFFFF)
+    return fail(MKV_ERR_UNSUPPORTED, "total_tokens too large");
 
   ShiftParams sp;
   memset(&sp, 0, sizeof sp);
@@ -1942,11 +1984,12 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   sp.layers = d->layers;
   sp.heads = d->heads;
   sp.rotary = d->rotary;
-  sp.tile_tokens = g.tile_tokens;
   sp.xcds = g.xcds;
   sp.chunks_per_row = g.chunks_per_row;
   sp.rows_per_wave = g.rows_per_wave;
+  sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
+  const int64_t tiles = set_tiles(g, d->total_tokens, sp);
 
   // one launch and no workspace: the shift kernel resolves every token from the span
   // table, the caller's token prefix and the caller's per-span tables
@@ -2133,8 +2176,8 @@ extern "C" int mkv_shift_spans_small(const mkv_shift_desc_t* d, void* stream) {
     return fail(MKV_ERR_UNSUPPORTED,
                 "a small shift needs power-of-two block sizes and heads a multiple of %d",
                 g.rows_per_wave);
-  const int64_t tiles = (d->total_tokens + g.tile_tokens - 1) / g.tile_tokens;
-  if (tiles > 0x7FFFFFFF) return fail(MKV_ERR_UNSUPPORTED, "total_tokens too large");
+  if ((d->total_tokens + g.tile_tokens - 1) / g.tile_tokens > 0x7FFFFFFF)
+    return fail(MKV_ERR_UNSUPPORTED, "total_tokens too large");
 
   static thread_local SmallParams a;  // ~2 KB: kept off the stack, rewritten every call
   memset(&a, 0, sizeof a);
@@ -2175,12 +2218,13 @@ extern "C" int mkv_shift_spans_small(const mkv_shift_desc_t* d, void* stream) {
   sp.layers = d->layers;
   sp.heads = d->heads;
   sp.rotary = d->rotary;
-  sp.tile_tokens = g.tile_tokens;
   sp.xcds = g.xcds;
   sp.chunks_per_row = g.chunks_per_row;
   sp.rows_per_wave = g.rows_per_wave;
+  sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
   sp.n_spans = d->n_spans;
+  const int64_t tiles = set_tiles(g, d->total_tokens, sp);
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (d->dtype) {
     case MKV_BF16:
