@@ -89,6 +89,10 @@
 #ifndef MKV_WG_THREADS
 #define MKV_WG_THREADS 128
 #endif
+// Workgroups of the one-layer kernel (mkv_scatter_shifted; see scatter_passes).
+#ifndef MKV_SINGLE_THREADS
+#define MKV_SINGLE_THREADS 256
+#endif
 // Plan pass: the per-span cos/sin tables are made by workgroups of their own, which need
 // no token prefix, instead of by the first record workgroups after their records' chain
 // (0.5 us less per two-launch call on 2,048-token and one-head shifts; 0: off).
@@ -210,13 +214,13 @@ namespace {
 
 constexpr int kThreads = MKV_WG_THREADS;  // shift kernel; a multiple of the 64-lane wave
 constexpr int kWaves = kThreads / 64;
+constexpr int kSingleThreads = MKV_SINGLE_THREADS;  // one span of one layer per launch
 
 // layers per workgroup of the record path (the direct path picks its own per launch)
-template <int DT, bool BATCHED, bool UNIFORM>
+template <int DT, bool UNIFORM>
 constexpr int layer_batch() {
-  return !BATCHED   ? 1
-         : UNIFORM ? MKV_LAYERS_RECORDS
-                   : (DT == MKV_FP8_E4M3 ? MKV_LAYERS_RECORDS_NU_1B : MKV_LAYERS_RECORDS_NU);
+  return UNIFORM ? MKV_LAYERS_RECORDS
+                 : (DT == MKV_FP8_E4M3 ? MKV_LAYERS_RECORDS_NU_1B : MKV_LAYERS_RECORDS_NU);
 }
 constexpr int kPlanThreads = 256;  // plan kernel
 // Buffer resources for the stores: raw (stride 0), the whole 32-bit range checked by
@@ -930,21 +934,21 @@ __global__ __launch_bounds__(kScatterThreads) void order_scatter_kernel(
 
 // -------------------------------------------------------------------- shift kernel
 //
-// Grid (token tiles, layer groups of LB layers).  Wave w of the workgroup runs passes
-// q = w + kWaves * u (u < U); pass q covers rows [q * rpw, (q + 1) * rpw) of the tile's
+// Grid (token tiles, layer groups of LB layers).  Wave w of the workgroup's W runs passes
+// q = w + W * u (u < U); pass q covers rows [q * rpw, (q + 1) * rpw) of the tile's
 // token-major (token, head) rows, in each of the workgroup's LB layers.  UNIFORM:
 // heads % rpw == 0, so every row of a pass belongs to one token.  BATCHED: a span
 // table (records from the plan pass, or DIRECT: resolved here); otherwise one span of
 // one layer (mkv_scatter_shifted).  SMALL: the span table and index windows are the
 // launch's arguments.
 
-template <int DT, bool BATCHED, bool UNIFORM, bool DIRECT, bool SMALL, int LB>
+template <int DT, bool BATCHED, bool UNIFORM, bool DIRECT, bool SMALL, int LB, int U, int T>
 __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack* q) {
   static_assert(!DIRECT || (BATCHED && UNIFORM), "direct shifts resolve one token per pass");
   static_assert(!SMALL || DIRECT, "small shifts take the direct path");
   using E = Elem<DT>;
   constexpr int C = E::kPerChunk;
-  constexpr int U = passes<DT, UNIFORM>();
+  constexpr int W = T / 64;  // waves of the workgroup
   static_assert(LB >= 1 && (BATCHED || LB == 1), "one layer per single-span launch");
   constexpr int N = U * LB;  // (pass, layer) units of one sweep: x = u * LB + lb
 
@@ -1069,7 +1073,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
       BATCHED && !UNIFORM && !SMALL && (MKV_TABLE_LDS & 4) != 0 && DT == MKV_FP8_E4M3;
   float* wave_tab = nullptr;
   if constexpr (kLdsTab || kLdsTabLanes) {
-    __shared__ __align__(16) float tab_lds[kWaves][2 * MKV_MAX_HEAD_SIZE];
+    __shared__ __align__(16) float tab_lds[W][2 * MKV_MAX_HEAD_SIZE];
     wave_tab = tab_lds[wave];
   }
   // stage span sp's [2][rotary] table (rotary / 2 chunks of 16 bytes) into the wave's LDS
@@ -1163,7 +1167,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
     if (p.rotary > 0) {
       const int half = p.rotary / 2;
       const int pairs = (small_hi - small_lo + 1) * half;
-      for (int idx = tid; idx < pairs; idx += kThreads) {
+      for (int idx = tid; idx < pairs; idx += T) {
         const int k = idx / half;
         const int f = idx - k * half;
         const int dl = q->spans[small_lo + k].delta;
@@ -1176,7 +1180,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
       __syncthreads();
     }
   }
-  for (int r0 = seg_row; r0 < nrows; r0 += kWaves * U * rpw) {
+  for (int r0 = seg_row; r0 < nrows; r0 += W * U * rpw) {
     // ---- phase A: where each pass reads and writes (uniform when UNIFORM).  All token
     // metadata is fetched first, then all base addresses, so the workgroup pays two
     // metadata round trips in total rather than two per pass; a token's metadata serves
@@ -1192,7 +1196,7 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
     int sb_u[U], db_u[U];      // the (group, layer 0) rows of the base tables
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int row0 = r0 + (MKV_PASS_MAJOR ? wave * U + u : wave + kWaves * u) * rpw;
+      const int row0 = r0 + (MKV_PASS_MAJOR ? wave * U + u : wave + W * u) * rpw;
       const int r = UNIFORM ? row0 : row0 + row_in_wave;
       const int rr = r < nrows ? r : nrows - 1;  // clamp: metadata reads stay in range
       const int t = H == 1 ? rr
@@ -1552,15 +1556,21 @@ __device__ __forceinline__ void shift_body(const ShiftParams& p, const SmallPack
   }
 }
 
-template <int DT, bool BATCHED, bool UNIFORM, bool DIRECT, int LB>
+template <int DT, bool UNIFORM, bool DIRECT, int LB>
 __global__ __launch_bounds__(kThreads) void shift_kernel(ShiftParams p) {
-  shift_body<DT, BATCHED, UNIFORM, DIRECT, false, LB>(p, nullptr);
+  shift_body<DT, true, UNIFORM, DIRECT, false, LB, passes<DT, UNIFORM>(), kThreads>(p, nullptr);
+}
+
+// One span of one layer (mkv_scatter_shifted), U passes a wave.
+template <int DT, bool UNIFORM, int U>
+__global__ __launch_bounds__(kSingleThreads) void scatter_kernel(ShiftParams p) {
+  shift_body<DT, false, UNIFORM, false, false, 1, U, kSingleThreads>(p, nullptr);
 }
 
 // A small shift: the span table, prefix and index windows arrive in the arguments.
 template <int DT>
 __global__ __launch_bounds__(kThreads) void shift_small_kernel(SmallParams a) {
-  shift_body<DT, true, true, true, true, 1>(a.p, &a.q);
+  shift_body<DT, true, true, true, true, 1, passes<DT, true>(), kThreads>(a.p, &a.q);
 }
 
 // --------------------------------------------------------------------- host side
@@ -1634,8 +1644,8 @@ int make_side(const mkv_side_t& in, int eb, DevSide& out, int64_t& hstride_b, co
 struct Geometry {
   int chunks_per_row;
   int rows_per_wave;
+  int sweep_rows;  // rows one sweep of a batched shift's workgroup covers
   int tile_tokens;
-  int sweep_rows;  // rows one sweep of a workgroup covers
   bool uniform;
   uint32_t heads_magic;
   int xcds;  // the tile order (MKV_XCD_MIN_TOKEN_BYTES)
@@ -1666,8 +1676,9 @@ int check_geometry(int dtype, int heads, int head_size, int rotary, int64_t src_
   const int rows = g.rows_per_wave * kWaves * passes_of(dtype, g.uniform);
   g.sweep_rows = rows;
   g.tile_tokens = rows / heads > 0 ? rows / heads : 1;
-  // row -> (token, head) uses a 32-bit reciprocal, exact while rows < 2^16
-  if (static_cast<int64_t>(g.tile_tokens) * heads >= (1 << 16))
+  // row -> (token, head) uses a 32-bit reciprocal, exact while a tile's rows < 2^16 (a
+  // sweep has at most 2^10)
+  if (heads >= (1 << 16))
     return fail(MKV_ERR_UNSUPPORTED, "heads %d too large", heads);
   g.heads_magic =
       heads == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + heads - 1) / heads);
@@ -1682,7 +1693,8 @@ int check_geometry(int dtype, int heads, int head_size, int rotary, int64_t src_
   return MKV_OK;
 }
 
-// The tiles of a shift of `tokens` tokens, and how they map to rows (sp's tile fields).
+// The tiles of a shift of `tokens` tokens by workgroups of `sweep_rows` rows, and how they
+// map to rows (sp's tile fields).
 //
 // A token of more rows than one sweep of a workgroup (2-byte elements: more than 8 KV
 // heads of 128, or 4 of 256) is cut into segments of one sweep, each a workgroup of its
@@ -1693,12 +1705,12 @@ int check_geometry(int dtype, int heads, int head_size, int rotary, int64_t src_
 // us, 40 one-layer launches of the latter 605 / 529 us.  A segment's number comes from a 32-bit
 // reciprocal; where that would not be exact over the grid (billions of segments), a
 // workgroup keeps the whole token.
-int64_t set_tiles(const Geometry& g, int64_t tokens, ShiftParams& sp) {
-  sp.tile_tokens = g.tile_tokens;
+int64_t set_tiles(int sweep_rows, int64_t tokens, ShiftParams& sp) {
+  sp.tile_tokens = sweep_rows / sp.heads > 0 ? sweep_rows / sp.heads : 1;
   sp.segs = 1;
   sp.segs_magic = 0;
   sp.sweep_rows = 1 << 16;  // a tile has fewer rows (check_geometry)
-  const int64_t segs = (sp.heads + g.sweep_rows - 1) / g.sweep_rows;
+  const int64_t segs = (sp.heads + sweep_rows - 1) / sweep_rows;
   if (segs > 1 && tokens <= 0x7FFFFFFF / segs - MKV_XCDS) {
     const uint64_t magic = ((uint64_t{1} << 32) + segs - 1) / segs;
     const uint64_t excess = magic * segs - (uint64_t{1} << 32);
@@ -1706,60 +1718,65 @@ int64_t set_tiles(const Geometry& g, int64_t tokens, ShiftParams& sp) {
     if (grid * excess < (uint64_t{1} << 32)) {
       sp.segs = static_cast<int32_t>(segs);
       sp.segs_magic = static_cast<uint32_t>(magic);
-      sp.sweep_rows = g.sweep_rows;
+      sp.sweep_rows = sweep_rows;
       return tokens * segs;
     }
   }
-  return (tokens + g.tile_tokens - 1) / g.tile_tokens;
+  return (tokens + sp.tile_tokens - 1) / sp.tile_tokens;
 }
 
-template <int DT, bool BATCHED, bool UNIFORM, bool DIRECT, int LB>
-int launch_shift(const ShiftParams& sp, int64_t tiles, int layers, hipStream_t stream) {
-  // tiles is rounded up to a multiple of MKV_XCDS below; extra workgroups exit at once
-  if (tiles <= 0) return MKV_OK;
+// The grid of `tiles` x `layer_groups` workgroups and the tile order, into q and `grid`.
+int set_grid(int64_t tiles, int layer_groups, ShiftParams& q, dim3& grid) {
+  // rounded up to a multiple of MKV_XCDS; extra workgroups exit at once
   tiles = (tiles + MKV_XCDS - 1) / MKV_XCDS * MKV_XCDS;
-  const int layer_groups = (layers + LB - 1) / LB;
   if (tiles > 0x7FFFFFFF || layer_groups > 65535)
     return fail(MKV_ERR_UNSUPPORTED, "grid of %lld x %d tiles too large", (long long)tiles,
                 layer_groups);
-  ShiftParams q = sp;
-  q.xcd_per = sp.xcds > 1 ? static_cast<int32_t>(tiles / MKV_XCDS) : 0;
-  q.layer_groups = 0;
-  dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(layer_groups));
-  if (BATCHED && !DIRECT && sp.layer_groups != 0 && tiles * layer_groups <= 0x7FFFFFFF) {
-    q.layer_groups = layer_groups;
-    grid = dim3(static_cast<unsigned>(tiles * layer_groups), 1);
-  }
-  hipLaunchKernelGGL((shift_kernel<DT, BATCHED, UNIFORM, DIRECT, LB>), grid, dim3(kThreads), 0,
-                     stream, q);
+  q.xcd_per = q.xcds > 1 ? static_cast<int32_t>(tiles / MKV_XCDS) : 0;
+  const bool layer_major = q.layer_groups != 0 && tiles * layer_groups <= 0x7FFFFFFF;
+  q.layer_groups = layer_major ? layer_groups : 0;
+  grid = layer_major ? dim3(static_cast<unsigned>(tiles * layer_groups), 1)
+                     : dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(layer_groups));
+  return MKV_OK;
+}
+
+template <typename Params>
+int launch(void (*kernel)(Params), dim3 grid, int threads, size_t lds, hipStream_t stream,
+           const Params& params) {
+  hipLaunchKernelGGL(kernel, grid, dim3(static_cast<unsigned>(threads)), lds, stream, params);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MKV_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
   return MKV_OK;
 }
 
+template <int DT, bool UNIFORM, bool DIRECT, int LB>
+int launch_shift(const ShiftParams& sp, int64_t tiles, int layers, hipStream_t stream) {
+  if (tiles <= 0) return MKV_OK;
+  ShiftParams q = sp;
+  dim3 grid;
+  const int rc = set_grid(tiles, (layers + LB - 1) / LB, q, grid);
+  if (rc != MKV_OK) return rc;
+  return launch(shift_kernel<DT, UNIFORM, DIRECT, LB>, grid, kThreads, 0, stream, q);
+}
+
 // direct_layers: the direct path's layers per workgroup (1, or MKV_DIRECT_WIDE_LAYERS for
 // a larger shift of 2-byte elements); 0 = the record path.
-template <bool BATCHED>
 int launch_any(int dtype, bool uniform, int direct_layers, const ShiftParams& sp,
                int64_t tiles, int layers, hipStream_t stream) {
-
 #define MKV_CASE(DT)                                                                        \
   case DT:                                                                                  \
-    if constexpr (BATCHED) {                                                                \
-      if (uniform && direct_layers > 0) {                                                   \
-        if constexpr (Elem<DT>::kBytes == 2 && MKV_DIRECT_WIDE_LAYERS > 1) {                \
-          if (direct_layers > 1)                                                            \
-            return launch_shift<DT, true, true, true, MKV_DIRECT_WIDE_LAYERS>(sp, tiles,    \
-                                                                              layers, stream); \
-        }                                                                                   \
-        return launch_shift<DT, true, true, true, 1>(sp, tiles, layers, stream);            \
+    if (uniform && direct_layers > 0) {                                                     \
+      if constexpr (Elem<DT>::kBytes == 2 && MKV_DIRECT_WIDE_LAYERS > 1) {                  \
+        if (direct_layers > 1)                                                              \
+          return launch_shift<DT, true, true, MKV_DIRECT_WIDE_LAYERS>(sp, tiles, layers,    \
+                                                                      stream);              \
       }                                                                                     \
+      return launch_shift<DT, true, true, 1>(sp, tiles, layers, stream);                    \
     }                                                                                       \
-    return uniform                                                                          \
-               ? launch_shift<DT, BATCHED, true, false, layer_batch<DT, BATCHED, true>()>(     \
-                     sp, tiles, layers, stream)                                             \
-               : launch_shift<DT, BATCHED, false, false, layer_batch<DT, BATCHED, false>()>(   \
-                     sp, tiles, layers, stream);
+    return uniform ? launch_shift<DT, true, false, layer_batch<DT, true>()>(sp, tiles,      \
+                                                                            layers, stream) \
+                   : launch_shift<DT, false, false, layer_batch<DT, false>()>(              \
+                         sp, tiles, layers, stream);
   switch (dtype) {
     MKV_CASE(MKV_BF16)
     MKV_CASE(MKV_F16)
@@ -1769,6 +1786,58 @@ int launch_any(int dtype, bool uniform, int direct_layers, const ShiftParams& sp
       return fail(MKV_ERR_DTYPE, "unknown dtype %d", dtype);
   }
 #undef MKV_CASE
+}
+
+// Passes a wave of a one-layer launch makes, by the waves the launch would have at one pass
+// each (`waves`, of 2 KB read and 2 KB written).  A launch this small is over in one or two
+// generations of resident waves, so its shape matters more than its inner loop: the fewest
+// passes that let every wave be resident at once with at most four waves on a SIMD (256
+// CUs of 4 SIMDs, and every variant's registers allow four; fp8's per-lane one, three).
+// Past that a launch takes several generations either way, and one pass overlaps loads and
+// stores best.  Measured, 40 launches back to back, us a launch at 1 / 2 / 4 passes (8
+// heads of 128; 256-thread workgroups, a few percent ahead of 128 wherever the passes
+// differ):
+//   bf16   8 MB (1,952 waves) 4.53 / 4.61 / 5.71   16 MB (3,906) 5.30 / 5.39 / 6.01
+//         33 MB (8,056) 7.67 / 7.12 / 7.71         50 MB (12,206) 10.63 / 9.65 / 9.70
+//         67 MB (16,356) 13.2 / 14.6 / 13.9        200 MB 34.1 / 36.7 / 39.6
+//   fp32  33 MB 7.54 / 7.23 / 7.62   50 MB 10.2 / 10.5 / 9.95   67 MB 12.7 / 13.9 / 12.8
+//   fp8   16 MB 6.87 / 6.22 / 7.40   50 MB 12.8 / 13.7 / 11.3   67 MB 15.7 / 16.3 / 13.9
+//   bf16, 2 heads: 42 MB 10.0 / 10.0 / 8.5, 50 MB 11.3 / 11.1 / 9.1, 67 MB 14.1 / 14.5 / 14.6
+constexpr int64_t kSimds = 1024;
+
+int scatter_passes(int dtype, const Geometry& g, int64_t tokens, int heads) {
+  const int64_t waves = (tokens * heads + g.rows_per_wave - 1) / g.rows_per_wave;
+  const bool fp8 = dtype == MKV_FP8_E4M3;
+  if (waves <= 3 * kSimds) return 1;
+  if (waves <= 2 * 4 * kSimds) return 2;
+  // (fp8's one-pass kernel holds fewer waves at once, so four passes win a little longer)
+  if (waves <= 4 * (fp8 && g.uniform ? 4 : 3) * kSimds) return 4;
+  return fp8 ? 2 : 1;
+}
+
+template <int DT, int U>
+int launch_scatter(const Geometry& g, const ShiftParams& sp, int64_t tokens,
+                   hipStream_t stream) {
+  ShiftParams q = sp;
+  const int64_t tiles = set_tiles(g.rows_per_wave * (kSingleThreads / 64) * U, tokens, q);
+  dim3 grid;
+  const int rc = set_grid(tiles, 1, q, grid);
+  if (rc != MKV_OK) return rc;
+  return g.uniform ? launch(scatter_kernel<DT, true, U>, grid, kSingleThreads, 0, stream, q)
+                   : launch(scatter_kernel<DT, false, U>, grid, kSingleThreads, 0, stream, q);
+}
+
+template <int DT>
+int launch_scatter_any(const Geometry& g, const ShiftParams& sp, int64_t tokens,
+                       hipStream_t stream) {
+  switch (scatter_passes(DT, g, tokens, sp.heads)) {
+    case 1:
+      return launch_scatter<DT, 1>(g, sp, tokens, stream);
+    case 2:
+      return launch_scatter<DT, 2>(g, sp, tokens, stream);
+    default:
+      return launch_scatter<DT, 4>(g, sp, tokens, stream);
+  }
 }
 
 int64_t workspace_bytes(int64_t total_tokens, int32_t n_spans, int32_t rotary) {
@@ -1935,9 +2004,17 @@ extern "C" int mkv_scatter_shifted(const void* src, int64_t src_token_stride,
   sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
   sp.rotate = rot ? 1 : 0;
-  const int64_t tiles = set_tiles(g, n_tokens, sp);
-  return launch_any<false>(dtype, g.uniform, 0, sp, tiles, 1,
-                           static_cast<hipStream_t>(stream));
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case MKV_BF16:
+      return launch_scatter_any<MKV_BF16>(g, sp, n_tokens, st);
+    case MKV_F16:
+      return launch_scatter_any<MKV_F16>(g, sp, n_tokens, st);
+    case MKV_F32:
+      return launch_scatter_any<MKV_F32>(g, sp, n_tokens, st);
+    default:
+      return launch_scatter_any<MKV_FP8_E4M3>(g, sp, n_tokens, st);
+  }
 }
 
 namespace {
@@ -1989,7 +2066,7 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   sp.rows_per_wave = g.rows_per_wave;
   sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
-  const int64_t tiles = set_tiles(g, d->total_tokens, sp);
+  const int64_t tiles = set_tiles(g.sweep_rows, d->total_tokens, sp);
 
   // one launch and no workspace: the shift kernel resolves every token from the span
   // table, the caller's token prefix and the caller's per-span tables
@@ -2012,7 +2089,7 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
         eb == 2 && d->total_tokens * d->layers > MKV_DIRECT_WIDE_MIN_ROWS
             ? MKV_DIRECT_WIDE_LAYERS
             : 1;
-    return launch_any<true>(d->dtype, true, direct_layers, sp, tiles, d->layers, st);
+    return launch_any(d->dtype, true, direct_layers, sp, tiles, d->layers, st);
   }
 
   if (d->order != MKV_ORDER_NONE && d->order != MKV_ORDER_DST_PAGE)
@@ -2113,22 +2190,17 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   sp.dst_hstride = dst_hs;
   sp.layer_groups = d->src.groups >= MKV_LAYER_MAJOR_MIN_GROUPS &&
                     d->total_tokens >= MKV_LAYER_MAJOR_MIN_TOKENS;
-  return launch_any<true>(d->dtype, g.uniform, 0, sp, tiles, d->layers, st);
+  return launch_any(d->dtype, g.uniform, 0, sp, tiles, d->layers, st);
 }
 
 template <int DT>
 int launch_small(SmallParams& a, int64_t tiles, int layers, hipStream_t stream) {
-  tiles = (tiles + MKV_XCDS - 1) / MKV_XCDS * MKV_XCDS;
-  if (tiles > 0x7FFFFFFF) return fail(MKV_ERR_UNSUPPORTED, "grid of %lld tiles too large", (long long)tiles);
-  a.p.xcd_per = a.p.xcds > 1 ? static_cast<int32_t>(tiles / MKV_XCDS) : 0;
+  dim3 grid;
+  const int rc = set_grid(tiles, layers, a.p, grid);
+  if (rc != MKV_OK) return rc;
   // LDS for the rotation tables of the spans one workgroup may touch
   const size_t lds = static_cast<size_t>(a.p.n_spans) * 2 * a.p.rotary * sizeof(float);
-  hipLaunchKernelGGL(shift_small_kernel<DT>,
-                     dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(layers)),
-                     dim3(kThreads), lds, stream, a);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(MKV_ERR_HIP, "launch failed: %s", hipGetErrorString(e));
-  return MKV_OK;
+  return launch(shift_small_kernel<DT>, grid, kThreads, lds, stream, a);
 }
 
 // One side's index window, from the caller's host array into the launch's int64 window.
@@ -2224,7 +2296,7 @@ extern "C" int mkv_shift_spans_small(const mkv_shift_desc_t* d, void* stream) {
   sp.lane_magic = (65536u + g.chunks_per_row - 1) / g.chunks_per_row;
   sp.heads_magic = g.heads_magic;
   sp.n_spans = d->n_spans;
-  const int64_t tiles = set_tiles(g, d->total_tokens, sp);
+  const int64_t tiles = set_tiles(g.sweep_rows, d->total_tokens, sp);
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (d->dtype) {
     case MKV_BF16:
