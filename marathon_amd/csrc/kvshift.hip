@@ -68,8 +68,13 @@
 #ifndef MKV_PASSES_2B
 #define MKV_PASSES_2B 1
 #endif
+// fp32, batched: one pass; more hold too many registers (four: 71 to 120 VGPRs against 30
+// to 52) and keep fewer waves resident.  One against four passes, whole calls, 40 layers: 4,096
+// tokens of 8 heads of 128 416 / 429 us, of 16 heads 839 / 873, 20,000 of one head 266 /
+// 292, a 300-token direct shift 38.0 / 45.6, a 2,000-token save 212 / 232, and 16 heads of
+// 256, 2,000 tokens, 831 / 910.
 #ifndef MKV_PASSES_4B
-#define MKV_PASSES_4B 4
+#define MKV_PASSES_4B 1
 #endif
 #ifndef MKV_PASSES_1B
 #define MKV_PASSES_1B 2
@@ -2084,7 +2089,8 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
     sp.n_spans = d->n_spans;
     sp.tables = d->span_tables;
     // several layers per workgroup only for 2-byte elements: fp8 would hold 16 rows' data
-    // across its two passes per wave, fp32 its four passes' (255 VGPRs, 2 waves per SIMD)
+    // across its two passes per wave, and fp32, whose rows are twice as long, measured
+    // 1-5% slower with four (300 tokens x 40 layers 39.3 against 38.0 us)
     const int direct_layers =
         eb == 2 && d->total_tokens * d->layers > MKV_DIRECT_WIDE_MIN_ROWS
             ? MKV_DIRECT_WIDE_LAYERS
