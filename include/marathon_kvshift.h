@@ -292,6 +292,28 @@ int mkv_shift_spans_small(const mkv_shift_desc_t* desc, void* stream);
 int mkv_shift_spans_noalloc(const mkv_shift_desc_t* desc, void* stream);
 #define MKV_NOALLOC_SCRATCH_BYTES (16LL << 20)
 
+/*
+ * The plan pass on the host, and the shift that takes its plan: for a short shift whose
+ * spans and indices are on the host, one launch and no per-token work on the device.
+ *
+ * mkv_plan_host (a host function, no GPU call) writes the plan of `desc` -- every token's
+ * source and destination row and the spans' rotation tables -- into desc->workspace.  Here
+ * desc->spans, inv_freq, src.index, dst.index, the sides' group_slots and workspace are
+ * HOST pointers; the base-address tables, k_scale, error_flags and the direct path's
+ * fields are not read.  The same rows, checks and table bits as the plan pass: a token
+ * whose index is out of range, or whose span's group is, gets an empty record and is not
+ * moved, and *flags (host, or NULL) receives the MKV_FLAG bits the device would have
+ * raised.  Span order only (order MKV_ORDER_NONE, no token_order).
+ *
+ * mkv_shift_spans_planned is mkv_shift_spans with desc->workspace (device) already
+ * holding that plan, copied there by the caller on the same stream: total_tokens, n_spans,
+ * layers, rotary, dtype and both sides' geometry must be those the plan was made with.
+ * desc->spans, inv_freq and the direct path's fields are ignored, and the sides' index
+ * and group_slots are not read.  Counterpart: mkv_shift_spans (same reference lines).
+ */
+int mkv_plan_host(const mkv_shift_desc_t* desc, int32_t* flags);
+int mkv_shift_spans_planned(const mkv_shift_desc_t* desc, void* stream);
+
 /* Workspace bytes mkv_shift_spans needs for these sizes (-1 on negative input). */
 int64_t mkv_shift_workspace_size(int64_t total_tokens, int32_t n_spans, int32_t rotary);
 
@@ -313,7 +335,7 @@ const char* mkv_last_error(void);
 
 /* ABI version of this header: (major << 16) | minor. */
 int32_t mkv_abi_version(void);
-#define MKV_ABI_VERSION ((3 << 16) | 4)
+#define MKV_ABI_VERSION ((3 << 16) | 5)
 
 #ifdef __cplusplus
 }

@@ -45,7 +45,7 @@ MKV_MAX_HEAD_SIZE = 512
 MKV_DIRECT_MAX_SPANS = 63
 MKV_SMALL_MAX_SPANS = 8
 MKV_SMALL_MAX_INDEX = 64
-MKV_ABI_VERSION = (3 << 16) | 4
+MKV_ABI_VERSION = (3 << 16) | 5
 MKV_ORDER_NONE = 0
 MKV_ORDER_DST_PAGE = 1
 MKV_NOALLOC_SCRATCH_BYTES = 16 << 20
@@ -64,6 +64,8 @@ EXPORTED = (
     "mkv_shift_spans",
     "mkv_shift_spans_noalloc",
     "mkv_shift_spans_small",
+    "mkv_plan_host",
+    "mkv_shift_spans_planned",
     "mkv_shift_workspace_size",
     "mkv_rope_tables",
     "mkv_last_error",
@@ -170,7 +172,8 @@ def _bind(cdll: ctypes.CDLL) -> ctypes.CDLL:
     f.restype = ctypes.c_int
     f.argtypes = [vp, i64, i64, vp, i64, i64, i64, i64, vp, i64, i32, i32, i32, i32, vp, vp,
                   i32, vp, vp, vp]
-    for name in ("mkv_shift_spans", "mkv_shift_spans_noalloc", "mkv_shift_spans_small"):
+    for name in ("mkv_shift_spans", "mkv_shift_spans_noalloc", "mkv_shift_spans_small",
+                 "mkv_plan_host", "mkv_shift_spans_planned"):
         f = getattr(cdll, name)
         f.restype = ctypes.c_int
         f.argtypes = [ctypes.POINTER(ShiftDesc), vp]

@@ -683,7 +683,7 @@ __device__ __forceinline__ void angle_cos_sin(int delta, float inv_freq_f, float
 
 // A span's table in the layout every path reads: [2][rotary], the cos of each element's
 // frequency, then its signed sine (-sin on the first half, +sin on the second).
-__device__ __forceinline__ void put_table(float* t, int rotary, int f, float c, float s) {
+__host__ __device__ __forceinline__ void put_table(float* t, int rotary, int f, float c, float s) {
   const int half = rotary / 2;
   t[f] = c;
   t[f + half] = c;
@@ -1845,6 +1845,32 @@ int launch_scatter_any(const Geometry& g, const ShiftParams& sp, int64_t tokens,
   }
 }
 
+// Span tables on the host.  The same operations whichever build of them runs: with the
+// FMA instruction (1.3 us a span of 64 frequencies; every x86 server of a decade has it) or
+// through the C library's fma() (4.8 us).
+__attribute__((always_inline)) inline void host_table_loop(int32_t delta, const float* inv_freq,
+                                                           int rotary, float* t) {
+  for (int f = 0; f < rotary / 2; ++f) {
+    float c, sn;
+    mkv_rope::angle_cos_sin(delta, inv_freq[f], c, sn);
+    put_table(t, rotary, f, c, sn);
+  }
+}
+
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+__attribute__((target("fma"), flatten)) void host_table_fma(int32_t delta, const float* inv_freq,
+                                                            int rotary, float* t) {
+  host_table_loop(delta, inv_freq, rotary, t);
+}
+#endif
+
+void host_table(int32_t delta, const float* inv_freq, int rotary, float* t) {
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+  if (__builtin_cpu_supports("fma")) return host_table_fma(delta, inv_freq, rotary, t);
+#endif
+  host_table_loop(delta, inv_freq, rotary, t);
+}
+
 int64_t workspace_bytes(int64_t total_tokens, int32_t n_spans, int32_t rotary) {
   return align256(static_cast<int64_t>(n_spans) * 2 * rotary *
                   static_cast<int64_t>(sizeof(float))) +
@@ -1915,18 +1941,8 @@ extern "C" int mkv_rope_tables(const int32_t* deltas, int32_t n_spans, const flo
   if (n_spans == 0 || rotary == 0) return MKV_OK;
   if (deltas == nullptr || inv_freq == nullptr || tables == nullptr)
     return fail(MKV_ERR_ARG, "null pointer");
-  const int half = rotary / 2;
-  for (int32_t sp = 0; sp < n_spans; ++sp) {
-    float* t = tables + static_cast<int64_t>(sp) * 2 * rotary;
-    for (int f = 0; f < half; ++f) {
-      float c, sn;
-      mkv_rope::angle_cos_sin(deltas[sp], inv_freq[f], c, sn);
-      t[f] = c;
-      t[f + half] = c;
-      t[rotary + f] = -sn;
-      t[rotary + f + half] = sn;
-    }
-  }
+  for (int32_t sp = 0; sp < n_spans; ++sp)
+    host_table(deltas[sp], inv_freq, rotary, tables + static_cast<int64_t>(sp) * 2 * rotary);
   return MKV_OK;
 }
 
@@ -2024,9 +2040,15 @@ extern "C" int mkv_scatter_shifted(const void* src, int64_t src_token_stride,
 
 namespace {
 
-// The batched shift.  noalloc: the workspace is this device's `scratch` array and the
-// descriptor's workspace fields are ignored.
-int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
+// Where the batched shift's plan comes from.
+enum PlanFrom {
+  kPlanDevice,   // the plan pass, into the descriptor's workspace
+  kPlanScratch,  // the plan pass, into this device's `scratch` array
+  kPlanHost      // the descriptor's workspace holds it already (mkv_plan_host): one launch
+};
+
+// The batched shift.
+int shift_spans(const mkv_shift_desc_t* d, void* stream, PlanFrom from) {
   g_err[0] = '\0';
   if (d == nullptr) return fail(MKV_ERR_ARG, "NULL descriptor");
   const int eb = elem_bytes(d->dtype);
@@ -2039,9 +2061,11 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
     return fail(MKV_ERR_UNSUPPORTED, "n_spans %d outside [0, %d]", d->n_spans, MKV_MAX_SPANS);
   if (d->total_tokens < 0) return fail(MKV_ERR_ARG, "total_tokens < 0");
   if (d->n_spans == 0 || d->total_tokens == 0) return MKV_OK;
-  if (d->spans == nullptr) return fail(MKV_ERR_ARG, "NULL span table");
+  const bool planned = from == kPlanHost;
+  if (d->spans == nullptr && !planned) return fail(MKV_ERR_ARG, "NULL span table");
   if (d->layers <= 0) return fail(MKV_ERR_ARG, "layers %d", d->layers);
-  if (d->rotary > 0 && d->inv_freq == nullptr) return fail(MKV_ERR_ARG, "inv_freq is NULL");
+  if (d->rotary > 0 && d->inv_freq == nullptr && !planned)
+    return fail(MKV_ERR_ARG, "inv_freq is NULL");
   if (d->dtype == MKV_FP8_E4M3 && d->rotary > 0 && d->k_scale == nullptr)
     return fail(MKV_ERR_ARG, "fp8 needs k_scale");
   if (d->src.k_base == nullptr || d->src.v_base == nullptr || d->dst.k_base == nullptr ||
@@ -2075,7 +2099,7 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
 
   // one launch and no workspace: the shift kernel resolves every token from the span
   // table, the caller's token prefix and the caller's per-span tables
-  if (d->span_starts != nullptr && d->span_tables != nullptr && g.uniform &&
+  if (!planned && d->span_starts != nullptr && d->span_tables != nullptr && g.uniform &&
       d->n_spans <= MKV_DIRECT_MAX_SPANS && ilog2_exact(d->src.block_size) >= 0 &&
       ilog2_exact(d->dst.block_size) >= 0) {
     if (!aligned16(reinterpret_cast<uint64_t>(d->span_tables)))
@@ -2101,11 +2125,13 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   if (d->order != MKV_ORDER_NONE && d->order != MKV_ORDER_DST_PAGE)
     return fail(MKV_ERR_ARG, "unknown order %d", d->order);
   const bool ordered = d->order == MKV_ORDER_DST_PAGE;
+  if (planned && (ordered || d->token_order != nullptr))
+    return fail(MKV_ERR_UNSUPPORTED, "a plan made on the host is in span order");
   const int64_t need = workspace_bytes(d->total_tokens, d->n_spans, d->rotary) +
                        (ordered ? MKV_ORDER_EXTRA_BYTES(d->total_tokens) : 0);
   void* ws_ptr = d->workspace;
   int64_t ws_bytes = d->workspace_bytes;
-  if (noalloc) {
+  if (from == kPlanScratch) {
     if (need > MKV_NOALLOC_SCRATCH_BYTES)
       return fail(MKV_ERR_UNSUPPORTED,
                   "this shift needs %lld bytes of workspace, more than the %lld bytes of "
@@ -2144,50 +2170,52 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   pp.layers = d->layers;
   pp.rotary = d->rotary;
 
-  const int64_t pairs = static_cast<int64_t>(d->n_spans) * (d->rotary / 2);
+  if (!planned) {
+    const int64_t pairs = static_cast<int64_t>(d->n_spans) * (d->rotary / 2);
 #if MKV_PLAN_TABLE_GROUPS
-  // record workgroups for the tokens, then table workgroups for the (span, frequency) pairs
-  const int64_t work = d->total_tokens;
-  int64_t tab_grid = (pairs + kPlanThreads - 1) / kPlanThreads;
-  if (tab_grid > 256) tab_grid = 256;
+    // record workgroups for the tokens, then table workgroups for the (span, frequency) pairs
+    const int64_t work = d->total_tokens;
+    int64_t tab_grid = (pairs + kPlanThreads - 1) / kPlanThreads;
+    if (tab_grid > 256) tab_grid = 256;
 #else
-  // every workgroup resolves records, then makes tables
-  const int64_t work = d->total_tokens > pairs ? d->total_tokens : pairs;
-  const int64_t tab_grid = 0;
+    // every workgroup resolves records, then makes tables
+    const int64_t work = d->total_tokens > pairs ? d->total_tokens : pairs;
+    const int64_t tab_grid = 0;
 #endif
-  int64_t plan_grid = (work + kPlanThreads - 1) / kPlanThreads;
-  if (plan_grid > 4096) plan_grid = 4096;
-  if (plan_grid < 1) plan_grid = 1;
-  TokRec* sorted = nullptr;
-  if (ordered) {  // sorted records, then the page counts, after the plan's records
-    int64_t groups = (d->total_tokens + kPlanThreads - 1) / kPlanThreads;
-    if (groups > kOrderMaxGroups) groups = kOrderMaxGroups;
-    if (groups < 1) groups = 1;
-    plan_grid = groups;
-    pp.order_chunk = (d->total_tokens + groups - 1) / groups;
-    sorted = recs + d->total_tokens;
-    pp.order_hist = reinterpret_cast<uint32_t*>(sorted + d->total_tokens);
-    // the destination's extent per (group, layer), in bytes, sets the bucket width
-    const int64_t cap = pp.dst.num_slots > 0 ? pp.dst.num_slots : 0;
-    const int64_t extent = (cap / pp.dst.block_size + 1) * pp.dst.bstride;
-    int shift = 21;
-    while (shift < 62 && (extent >> shift) >= kOrderBuckets) ++shift;
-    pp.order_shift = shift;
-  }
-  const size_t lds = sizeof(int64_t) * (static_cast<size_t>(d->n_spans) + 1);
-  pp.rec_groups = static_cast<int32_t>(plan_grid);  // the order kernel's groups too
-  hipLaunchKernelGGL(plan_kernel, dim3(static_cast<unsigned>(plan_grid + tab_grid)),
-                     dim3(kPlanThreads), lds, st, pp);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(MKV_ERR_HIP, "plan launch failed: %s", hipGetErrorString(e));
-  if (ordered) {
-    hipLaunchKernelGGL(order_scatter_kernel, dim3(static_cast<unsigned>(plan_grid)),
-                       dim3(kScatterThreads), 0, st, recs, sorted, pp.order_hist,
-                       d->total_tokens, pp.order_chunk, static_cast<int>(plan_grid),
-                       pp.order_shift);
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(MKV_ERR_HIP, "order launch failed: %s", hipGetErrorString(e));
-    recs = sorted;
+    int64_t plan_grid = (work + kPlanThreads - 1) / kPlanThreads;
+    if (plan_grid > 4096) plan_grid = 4096;
+    if (plan_grid < 1) plan_grid = 1;
+    TokRec* sorted = nullptr;
+    if (ordered) {  // sorted records, then the page counts, after the plan's records
+      int64_t groups = (d->total_tokens + kPlanThreads - 1) / kPlanThreads;
+      if (groups > kOrderMaxGroups) groups = kOrderMaxGroups;
+      if (groups < 1) groups = 1;
+      plan_grid = groups;
+      pp.order_chunk = (d->total_tokens + groups - 1) / groups;
+      sorted = recs + d->total_tokens;
+      pp.order_hist = reinterpret_cast<uint32_t*>(sorted + d->total_tokens);
+      // the destination's extent per (group, layer), in bytes, sets the bucket width
+      const int64_t cap = pp.dst.num_slots > 0 ? pp.dst.num_slots : 0;
+      const int64_t extent = (cap / pp.dst.block_size + 1) * pp.dst.bstride;
+      int shift = 21;
+      while (shift < 62 && (extent >> shift) >= kOrderBuckets) ++shift;
+      pp.order_shift = shift;
+    }
+    const size_t lds = sizeof(int64_t) * (static_cast<size_t>(d->n_spans) + 1);
+    pp.rec_groups = static_cast<int32_t>(plan_grid);  // the order kernel's groups too
+    hipLaunchKernelGGL(plan_kernel, dim3(static_cast<unsigned>(plan_grid + tab_grid)),
+                       dim3(kPlanThreads), lds, st, pp);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(MKV_ERR_HIP, "plan launch failed: %s", hipGetErrorString(e));
+    if (ordered) {
+      hipLaunchKernelGGL(order_scatter_kernel, dim3(static_cast<unsigned>(plan_grid)),
+                         dim3(kScatterThreads), 0, st, recs, sorted, pp.order_hist,
+                         d->total_tokens, pp.order_chunk, static_cast<int>(plan_grid),
+                         pp.order_shift);
+      e = hipGetLastError();
+      if (e != hipSuccess) return fail(MKV_ERR_HIP, "order launch failed: %s", hipGetErrorString(e));
+      recs = sorted;
+    }
   }
 
   sp.recs = recs;
@@ -2197,6 +2225,93 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, bool noalloc) {
   sp.layer_groups = d->src.groups >= MKV_LAYER_MAJOR_MIN_GROUPS &&
                     d->total_tokens >= MKV_LAYER_MAJOR_MIN_TOKENS;
   return launch_any(d->dtype, g.uniform, 0, sp, tiles, d->layers, st);
+}
+
+// ------------------------------------------------------------------ the plan on the host
+//
+// What plan_kernel writes into the workspace, by the CPU: a short shift whose spans and
+// indices are on the host needs no plan pass ahead of its shift kernel, and no resolving
+// inside it.  Runs of one block share their block's address, so a record costs about its
+// own 32 bytes of stores.
+
+int64_t wrap_add(int64_t a, int64_t b) {
+  return static_cast<int64_t>(static_cast<uint64_t>(a) + static_cast<uint64_t>(b));
+}
+
+// put(i, byte offset) for each of a span's tokens [0, n) whose index on this side is in
+// range, by resolve()'s rules; false if any is not.
+template <typename Put>
+bool host_rows(const DevSide& sd, int64_t cap, int64_t pos0, int64_t index0, int64_t n, Put put) {
+  const int64_t bs = sd.block_size;
+  bool all = true;
+  if (sd.mode == MKV_ADDR_SLOTS) {
+    const int64_t* slots = static_cast<const int64_t*>(sd.index);
+    for (int64_t i = 0; i < n; ++i) {
+      const int64_t ii = wrap_add(index0, i);
+      const int64_t slot = ii >= 0 && ii < sd.index_len ? slots[ii] : -1;
+      if (slot < 0 || slot >= cap) {
+        all = false;
+        continue;
+      }
+      const int64_t blk = sd.bs_shift >= 0 ? slot >> sd.bs_shift : slot / bs;
+      put(i, blk * sd.bstride + (slot - blk * bs) * sd.ostride);
+    }
+    return all;
+  }
+  const bool table = sd.mode == MKV_ADDR_TABLE;
+  const int64_t blocks = cap / bs;
+  for (int64_t i = 0; i < n;) {
+    const int64_t pos = wrap_add(pos0, i);
+    if (pos < 0) {
+      all = false;
+      ++i;
+      continue;
+    }
+    int64_t blk = sd.bs_shift >= 0 ? pos >> sd.bs_shift : pos / bs;
+    const int64_t off = pos - blk * bs;
+    int64_t run = bs - off < n - i ? bs - off : n - i;  // tokens of this block
+    bool ok;
+    if (table) {
+      const int64_t ti = wrap_add(index0, blk);
+      ok = ti >= 0 && ti < sd.index_len;
+      if (ok) {
+        blk = static_cast<const int32_t*>(sd.index)[ti];
+        ok = blk >= 0 && blk < blocks;
+      }
+    } else {
+      ok = pos < cap;
+      if (ok && cap - pos < run) run = cap - pos;
+    }
+    if (ok) {
+      int64_t at = blk * sd.bstride + off * sd.ostride;
+      for (int64_t k = 0; k < run; ++k, at += sd.ostride) put(i + k, at);
+    } else {
+      all = false;
+    }
+    i += run;
+  }
+  return all;
+}
+
+constexpr int64_t kNoRow = INT64_MIN;  // a token whose index is out of range
+
+// The records of span `s`'s first n tokens; returns the flags the plan pass would raise.
+int32_t host_records(const mkv_shift_desc_t* d, const DevSide& src, const DevSide& dst, int s,
+                     int64_t n, TokRec* recs) {
+  const mkv_span_t& sp = d->spans[s];
+  const TokRec start = {kNoRow, kNoRow, s, sp.delta, sp.src_group * d->layers, sp.dst_group * d->layers};
+  for (int64_t i = 0; i < n; ++i) recs[i] = start;
+  const int64_t s_cap = src.group_slots != nullptr ? src.group_slots[sp.src_group] : src.num_slots;
+  const int64_t d_cap = dst.group_slots != nullptr ? dst.group_slots[sp.dst_group] : dst.num_slots;
+  const bool s_ok = host_rows(src, s_cap, sp.src_pos, sp.src_index, n,
+                              [&](int64_t i, int64_t off) { recs[i].src_off = off; });
+  const bool d_ok = host_rows(dst, d_cap, sp.dst_pos, sp.dst_index, n,
+                              [&](int64_t i, int64_t off) { recs[i].dst_off = off; });
+  if (!s_ok || !d_ok) {
+    for (int64_t i = 0; i < n; ++i)
+      if (recs[i].src_off == kNoRow || recs[i].dst_off == kNoRow) recs[i] = TokRec{0, 0, -1, 0, 0, 0};
+  }
+  return (s_ok ? 0 : MKV_FLAG_SRC_RANGE) | (d_ok ? 0 : MKV_FLAG_DST_RANGE);
 }
 
 template <int DT>
@@ -2225,7 +2340,7 @@ int pack_index(const mkv_side_t& in, int64_t* out, const char* name) {
 }  // namespace
 
 extern "C" int mkv_shift_spans(const mkv_shift_desc_t* d, void* stream) {
-  return shift_spans(d, stream, false);
+  return shift_spans(d, stream, kPlanDevice);
 }
 
 extern "C" int mkv_shift_spans_small(const mkv_shift_desc_t* d, void* stream) {
@@ -2317,5 +2432,69 @@ extern "C" int mkv_shift_spans_small(const mkv_shift_desc_t* d, void* stream) {
 }
 
 extern "C" int mkv_shift_spans_noalloc(const mkv_shift_desc_t* d, void* stream) {
-  return shift_spans(d, stream, true);
+  return shift_spans(d, stream, kPlanScratch);
+}
+
+extern "C" int mkv_shift_spans_planned(const mkv_shift_desc_t* d, void* stream) {
+  return shift_spans(d, stream, kPlanHost);
+}
+
+extern "C" int mkv_plan_host(const mkv_shift_desc_t* d, int32_t* flags) {
+  g_err[0] = '\0';
+  if (flags != nullptr) *flags = 0;
+  if (d == nullptr) return fail(MKV_ERR_ARG, "NULL descriptor");
+  const int eb = elem_bytes(d->dtype);
+  if (eb == 0) return fail(MKV_ERR_DTYPE, "unknown dtype %d", d->dtype);
+  if (d->n_spans < 0 || d->n_spans > MKV_MAX_SPANS)
+    return fail(MKV_ERR_UNSUPPORTED, "n_spans %d outside [0, %d]", d->n_spans, MKV_MAX_SPANS);
+  if (d->total_tokens < 0) return fail(MKV_ERR_ARG, "total_tokens < 0");
+  if (d->rotary < 0 || d->rotary % 2 != 0) return fail(MKV_ERR_ARG, "rotary %d", d->rotary);
+  if (d->layers <= 0) return fail(MKV_ERR_ARG, "layers %d", d->layers);
+  if (d->n_spans == 0 || d->total_tokens == 0) return MKV_OK;
+  if (d->spans == nullptr) return fail(MKV_ERR_ARG, "NULL span table");
+  if (d->rotary > 0 && d->inv_freq == nullptr) return fail(MKV_ERR_ARG, "inv_freq is NULL");
+  if (d->order != MKV_ORDER_NONE || d->token_order != nullptr)
+    return fail(MKV_ERR_UNSUPPORTED, "a plan made on the host is in span order");
+  const int64_t need = workspace_bytes(d->total_tokens, d->n_spans, d->rotary);
+  if (d->workspace == nullptr || d->workspace_bytes < need)
+    return fail(MKV_ERR_ARG, "workspace of %lld bytes needed (mkv_shift_workspace_size)",
+                (long long)need);
+  if (!aligned16(reinterpret_cast<uint64_t>(d->workspace)))
+    return fail(MKV_ERR_ALIGN, "workspace not 16-byte aligned");
+  DevSide src, dst;
+  int64_t hs = 0;
+  int rc = make_side(d->src, eb, src, hs, "src");
+  if (rc != MKV_OK) return rc;
+  rc = make_side(d->dst, eb, dst, hs, "dst");
+  if (rc != MKV_OK) return rc;
+
+  float* tables = static_cast<float*>(d->workspace);
+  TokRec* recs = reinterpret_cast<TokRec*>(static_cast<char*>(d->workspace) + need) -
+                 d->total_tokens;
+  int32_t raised = 0;
+  int64_t at = 0;
+  for (int s = 0; s < d->n_spans; ++s) {
+    const mkv_span_t& sp = d->spans[s];
+    const bool groups_ok = sp.src_group >= 0 && sp.src_group < src.groups &&
+                           sp.dst_group >= 0 && sp.dst_group < dst.groups;
+    int64_t n = sp.n_tokens > 0 ? sp.n_tokens : 0;
+    if (!groups_ok || sp.n_tokens < 0) raised |= MKV_FLAG_SPAN;
+    if (n > d->total_tokens - at) {  // tokens beyond total_tokens are not moved
+      n = d->total_tokens - at;
+      raised |= MKV_FLAG_SPAN;
+    }
+    if (groups_ok) {
+      raised |= host_records(d, src, dst, s, n, recs + at);
+      if (n > 0 && sp.delta != 0) {  // an unmoved span's table is never read
+        host_table(sp.delta, d->inv_freq, d->rotary,
+                   tables + static_cast<int64_t>(s) * 2 * d->rotary);
+      }
+    } else {
+      for (int64_t i = 0; i < n; ++i) recs[at + i] = TokRec{0, 0, -1, 0, 0, 0};
+    }
+    at += n;
+  }
+  for (; at < d->total_tokens; ++at) recs[at] = TokRec{0, 0, -1, 0, 0, 0};
+  if (flags != nullptr) *flags = raised;
+  return MKV_OK;
 }

@@ -45,6 +45,13 @@ DIRECT_MAX_TOKEN_LAYERS = 20480
 #: workgroup then reads the arguments, which costs more than the copy from about 64
 #: tokens x 40 layers on (12.6 against 9.6 us of GPU time; 34 against 22 at 256).
 SMALL_ARGS_MAX_TOKEN_LAYERS = 2560
+#: SmallShifts plans a step on the host where its plan is at most this many bytes: a host
+#: copy of up to 16 KB is a small kernel on the stream (2.3 us), a larger one goes through a
+#: copy engine that the stream waits for, longer than for the 5.4 us plan pass it replaces.
+#: Loads of 36 layers, calls back to back, us, plan pass / host plan: bf16 303 tokens 51 /
+#: 31, 400 tokens 50 / 31, fp8 54 / 34; past 16 KB bf16 600 tokens 44 / 53, 800 tokens 53 /
+#: 62, fp8 37 / 43, 1,500 tokens 53 / 63.
+HOST_PLAN_MAX_BYTES = 16384
 
 
 #: Token orders of the two-launch path.  ``"dst_page"``: tokens sorted by the page of their
@@ -231,6 +238,7 @@ class CacheSet:
             blob = stage.upload(device)
             ready = torch.cuda.Event()
             ready.record()
+            self.upload_stream = current_stream(device)
             base = blob.data_ptr()
             got = self._dev = (base + offs[0], base + offs[1],
                                None if offs[2] is None else base + offs[2], ready, blob)
@@ -560,20 +568,22 @@ class ShiftPlan:
 
 
 class SmallShifts:
-    """Direct-path shifts of a few tokens, with no per-step allocation or descriptor
-    building: the steady state of a serving loop (a decode step's saves, short loads).
+    """Shifts with no :class:`ShiftPlan` to build: the steady state of a serving loop (a
+    decode step's saves, a prefill chunk's save, a step's loads).
 
-    One device buffer per (source caches, destination caches, addressing modes) holds a
-    step's span table, token prefix, rotation tables and index windows; :meth:`run`
-    rewrites it with one pinned copy on the current stream and launches the step with a
-    descriptor kept from the previous one.  Stream order keeps a step's copy after the
-    previous step's kernel, which still reads the buffer.  Only steps that take the
-    library's direct path come here (:meth:`fits`); the rest build a :class:`ShiftPlan`.
+    One runner per (source caches, destination caches, addressing modes) keeps the
+    descriptors.  :meth:`run` takes a step's spans and host indices to the GPU in one of
+    three ways:
+
+    * in the launch's own arguments, for a few tokens (``mkv_shift_spans_small``);
+    * as a plan made here (``mkv_plan_host``), copied to the device and launched alone
+      (``mkv_shift_spans_planned``), where the plan fits :data:`HOST_PLAN_MAX_BYTES`;
+    * as they are, in one pinned copy, for the plan pass and the shift (whole calls against
+      the direct path and its tables: 511 tokens x 40 layers, bf16 51 -> 41 us, fp8 54 ->
+      35; 200 tokens of 12 spans 94 -> 68; 20,000 tokens of one layer 55 -> 40).
+
+    Copies and launches go to the current stream; a step's device buffers are its own.
     """
-
-    SPANS_AT = 0
-    STARTS_AT = _lib.MKV_DIRECT_MAX_SPANS * _lib.SPAN_DTYPE.itemsize  # 3,024 B
-    TABLES_AT = STARTS_AT + 64 * 8
 
     def __init__(self, src: CacheSet, dst: CacheSet, *, inv_freq: torch.Tensor | None,
                  src_mode: str, dst_mode: str, k_scale: torch.Tensor | None = None):
@@ -593,8 +603,9 @@ class SmallShifts:
                          for m in (src_mode, dst_mode)]
         self._h_addr = (self._h_spans.ctypes.data, self._h_index[0].ctypes.data,
                         self._h_index[1].ctypes.data)
-        self.capacity = 0
-        self.buf = None
+        self._flags = np.zeros(1, np.int32)  # mkv_plan_host's
+        self._flags_at = self._flags.ctypes.data
+        self.buf = self.workspace = None  # the last step's, on the device
         self._keep = []
         with _on(self.device, self.device.index == torch.cuda.current_device()):
             static = _Staging()
@@ -609,7 +620,13 @@ class SmallShifts:
                 scale_off = static.add(scale)
             blob = static.upload(self.device)
             self._keep.append(blob)
-            sides = [cs.device_tables(self.device)[:3] for cs in (src, dst)]
+            tables = [cs.device_tables(self.device) for cs in (src, dst)]
+            self._build_stream = current_stream(self.device)
+        sides = [t[:3] for t in tables]
+        self._ready = [t[3] for t in tables]
+        # streams that need not wait for these uploads
+        self._synced = {self._build_stream} if all(
+            cs.upload_stream == self._build_stream for cs in (src, dst)) else set()
         base = blob.data_ptr()
         d = self.desc = _lib.ShiftDesc()
         d.inv_freq = None if inv_off is None else base + inv_off
@@ -621,21 +638,22 @@ class SmallShifts:
         # the same shift for mkv_shift_spans_small: host span rows and index windows
         self.small_desc = _lib.ShiftDesc()
         ctypes.memmove(ctypes.byref(self.small_desc), ctypes.byref(d), ctypes.sizeof(d))
+        # and for mkv_shift_spans: a step's own device copies of both
+        self.stage_desc = _lib.ShiftDesc()
+        ctypes.memmove(ctypes.byref(self.stage_desc), ctypes.byref(d), ctypes.sizeof(d))
+        self._now = d
+        # what mkv_plan_host reads, host addresses only
+        h = self.plan_desc = _lib.ShiftDesc()
+        ctypes.memmove(ctypes.byref(h), ctypes.byref(d), ctypes.sizeof(d))
+        h.inv_freq = None if inv_freq is None else self.inv_host.data_ptr()
+        for side, cs in ((h.src, src), (h.dst, dst)):
+            caps, uniform = cs.base_tables()[2], cs.base_tables()[4]
+            side.group_slots = None if uniform else caps.ctypes.data
         self._last: tuple = ()
         self.tokens = 0
 
     def fits(self, n_spans: int, tokens: int) -> bool:
-        return (self.eligible_geometry and 0 < n_spans <= _lib.MKV_DIRECT_MAX_SPANS
-                and tokens * self.dst.layers <= DIRECT_MAX_TOKEN_LAYERS)
-
-    def _ensure(self, nbytes: int) -> None:
-        if nbytes > self.capacity:
-            self.capacity = max(nbytes, 2 * self.capacity, self.TABLES_AT + 4096)
-            self.buf = torch.empty(self.capacity, dtype=torch.uint8, device=self.device)
-            base = self.buf.data_ptr()
-            self.desc.spans = base + self.SPANS_AT
-            self.desc.span_starts = base + self.STARTS_AT
-            self.desc.span_tables = base + self.TABLES_AT
+        return 0 < n_spans <= _lib.MKV_MAX_SPANS and tokens > 0
 
     def run(self, rows: list, src_index: np.ndarray | None, dst_index: np.ndarray | None,
             error_flags: torch.Tensor | None = None) -> None:
@@ -644,14 +662,13 @@ class SmallShifts:
 
         Up to ``MKV_SMALL_MAX_SPANS`` spans and ``MKV_SMALL_MAX_INDEX`` index entries a
         side, the rows and windows travel in the launch itself
-        (``mkv_shift_spans_small``); beyond that they are copied into this runner's
-        device buffer first."""
+        (``mkv_shift_spans_small``)."""
         n = len(rows)
         n_src = 0 if src_index is None else src_index.size
         n_dst = 0 if dst_index is None else dst_index.size
         tokens = sum(max(int(r[4]), 0) for r in rows)
-        if (n <= _lib.MKV_SMALL_MAX_SPANS and n_src <= _lib.MKV_SMALL_MAX_INDEX
-                and n_dst <= _lib.MKV_SMALL_MAX_INDEX
+        if (self.eligible_geometry and n <= _lib.MKV_SMALL_MAX_SPANS
+                and n_src <= _lib.MKV_SMALL_MAX_INDEX and n_dst <= _lib.MKV_SMALL_MAX_INDEX
                 and tokens * self.dst.layers <= SMALL_ARGS_MAX_TOKEN_LAYERS):
             hs = self._h_spans
             for i, r in enumerate(rows):
@@ -672,59 +689,101 @@ class SmallShifts:
             self.launch(error_flags=error_flags)
             return
         self._last = ()
-        spans = np.array(rows, dtype=_lib.SPAN_DTYPE)
-        counts = np.maximum(spans["n_tokens"], 0).astype(np.int64)
-        starts = np.zeros(n + 1, np.int64)
-        np.cumsum(counts, out=starts[1:])
-        src_t, src_b = self._idx[self.modes[0]]
-        dst_t, dst_b = self._idx[self.modes[1]]
-        # layout: span rows, prefix, the rotated spans' tables (when any), the indices
-        tables = None
-        if self.rotary and bool(spans["delta"].any()):
-            tables = span_tables(spans["delta"], self.inv_host, self.rotary)
-        src_at = self.TABLES_AT + (0 if tables is None else (tables.nbytes + 15) // 16 * 16)
-        dst_at = src_at + (n_src * src_b + 15) // 16 * 16
-        end = dst_at + n_dst * dst_b
-        self._ensure(end)
-        host = torch.empty(end, dtype=torch.uint8, pin_memory=True)
-        hv = host.numpy()
-        hv[self.SPANS_AT:self.SPANS_AT + spans.nbytes] = spans.view(np.uint8)
-        hv[self.STARTS_AT:self.STARTS_AT + starts.nbytes] = starts.view(np.uint8)
-        if tables is not None:
-            hv[self.TABLES_AT:self.TABLES_AT + tables.nbytes] = tables.reshape(-1).view(np.uint8)
-        if n_src:
-            hv[src_at:src_at + n_src * src_b] = np.ascontiguousarray(
-                src_index, dtype=src_t).view(np.uint8)
-        if n_dst:
-            hv[dst_at:dst_at + n_dst * dst_b] = np.ascontiguousarray(
-                dst_index, dtype=dst_t).view(np.uint8)
-        # one copy of the step's region (the gaps between parts are never read)
-        self.buf[:end].copy_(host, non_blocking=True)
-        d = self.desc
-        base = self.buf.data_ptr()
-        d.src.index = base + src_at if n_src else None
-        d.src.index_len = n_src
-        d.dst.index = base + dst_at if n_dst else None
-        d.dst.index_len = n_dst
-        d.n_spans = n
-        d.total_tokens = self.tokens = int(starts[-1])
+        self.tokens = tokens
+        # mkv_shift_workspace_size: the spans' tables, then 32 bytes a token
+        size = (n * 8 * self.rotary + 255) // 256 * 256 + 32 * tokens
+        rows = np.array(rows, dtype=_lib.SPAN_DTYPE)
+        if size <= HOST_PLAN_MAX_BYTES:
+            raised = self._plan_here(rows, src_index, dst_index, tokens, size)
+            if raised and error_flags is not None:
+                error_flags.bitwise_or_(raised)
+        else:
+            self._stage(rows, src_index, dst_index, tokens, size)
         self.launch(error_flags=error_flags)
 
+    def _upload(self, host: torch.Tensor) -> int:
+        """A pinned buffer's copy on the device, in a buffer of this step's own (the
+        allocator hands it on in stream order)."""
+        self.buf = torch.empty(host.numel(), dtype=torch.uint8, device=self.device)
+        self.buf.copy_(host, non_blocking=True)
+        return self.buf.data_ptr()
+
+    def _plan_here(self, spans: np.ndarray, src_index, dst_index, tokens: int,
+                   size: int) -> int:
+        """Plan the step on the host; returns the flags of rows that will not be moved."""
+        h = self.plan_desc
+        h.spans, h.n_spans, h.total_tokens = spans.ctypes.data, spans.size, tokens
+        windows = []  # alive until the call has read them
+        for side, mode, index in ((h.src, self.modes[0], src_index),
+                                  (h.dst, self.modes[1], dst_index)):
+            if index is None or index.size == 0:
+                side.index, side.index_len = None, 0
+                continue
+            index = np.ascontiguousarray(index, dtype=self._idx[mode][0])
+            windows.append(index)
+            side.index, side.index_len = index.ctypes.data, index.size
+        host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+        h.workspace, h.workspace_bytes = host.data_ptr(), size
+        _lib.check(_lib.lib().mkv_plan_host(ctypes.byref(h), self._flags_at))
+        d = self._now = self.desc
+        d.n_spans, d.total_tokens = spans.size, tokens
+        d.workspace, d.workspace_bytes = self._upload(host), size
+        return int(self._flags[0])
+
+    def _stage(self, spans: np.ndarray, src_index, dst_index, tokens: int, size: int) -> None:
+        """Copy the step's spans and indices to the device, for the plan pass there."""
+        parts, end = [spans], spans.nbytes
+        at = [None, None]
+        for k, (mode, index) in enumerate(zip(self.modes, (src_index, dst_index))):
+            if index is not None and index.size:
+                at[k] = end = (end + 15) // 16 * 16
+                parts.append(np.ascontiguousarray(index, dtype=self._idx[mode][0]))
+                end += parts[-1].nbytes
+        host = torch.empty(end, dtype=torch.uint8, pin_memory=True)
+        view = host.numpy()
+        for lo, a in zip([0] + [x for x in at if x is not None], parts):
+            view[lo:lo + a.nbytes] = a.reshape(-1).view(np.uint8)
+        base = self._upload(host)
+        d = self._now = self.stage_desc
+        d.spans, d.n_spans, d.total_tokens = base, spans.size, tokens
+        for side, lo, index in ((d.src, at[0], src_index), (d.dst, at[1], dst_index)):
+            side.index = None if lo is None else base + lo
+            side.index_len = 0 if lo is None else index.size
+        self.workspace = torch.empty(size, dtype=torch.uint8, device=self.device)
+        d.workspace, d.workspace_bytes = self.workspace.data_ptr(), size
+
     def launch(self, stream: int | None = None, error_flags: torch.Tensor | None = None) -> None:
-        """(Re)launch the last step on ``stream`` (default: current); a step that went
-        through the device buffer must run on the stream it was copied on."""
-        small = bool(self._last)
-        d = self.small_desc if small else self.desc
-        d.error_flags = None if error_flags is None else error_flags.data_ptr()
+        """(Re)launch the last step on ``stream`` (default: current); a step that copied
+        anything to the device must run on the stream it was copied on."""
+        if self.device.index != torch.cuda.current_device():
+            with torch.cuda.device(self.device):  # launches go to the current device
+                return self.launch(stream, error_flags)
         if stream is None:
             stream = current_stream(self.device)
+        stream = int(stream)
+        if stream not in self._synced:
+            self._sync(stream)
         L = _lib.lib()
-        fn = L.mkv_shift_spans_small if small else L.mkv_shift_spans
-        _lib.check(fn(ctypes.byref(d), ctypes.c_void_p(int(stream))))
+        if self._last:
+            d, fn = self.small_desc, L.mkv_shift_spans_small
+        elif self._now is self.desc:
+            d, fn = self.desc, L.mkv_shift_spans_planned
+        else:
+            d, fn = self._now, L.mkv_shift_spans
+        d.error_flags = None if error_flags is None else error_flags.data_ptr()
+        _lib.check(fn(ctypes.byref(d), stream))
 
-    @property
-    def direct(self) -> bool:
-        return True
+    def _sync(self, stream: int) -> None:
+        """A stream's first launch waits for what other streams uploaded: the caches'
+        base-address tables and this runner's frequencies and scales."""
+        ext = torch.cuda.ExternalStream(stream, device=self.device)
+        if not torch.cuda.is_current_stream_capturing():
+            ext.wait_stream(torch.cuda.ExternalStream(self._build_stream, device=self.device))
+            for ready in self._ready:
+                ext.wait_event(ready)
+        for t in self._keep:
+            t.record_stream(ext)
+        self._synced.add(stream)
 
     @property
     def algorithmic_bytes(self) -> int:
