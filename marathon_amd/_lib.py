@@ -164,6 +164,7 @@ class KVShiftError(RuntimeError):
 
 _LOCK = threading.Lock()
 _LIB: ctypes.CDLL | None = None
+_BINDING = None
 
 
 def _bind(cdll: ctypes.CDLL) -> ctypes.CDLL:
@@ -214,6 +215,30 @@ def lib() -> ctypes.CDLL:
                 raise RuntimeError("libmarathon_kvshift ABI version mismatch; rebuild")
             _LIB = cdll
     return _LIB
+
+
+def binding():
+    """The CPython module (``csrc/binding.cpp``), bound to the library; like :func:`lib`,
+    it raises if it has not been built."""
+    global _BINDING
+    if _BINDING is None:
+        cdll = lib()
+        with _LOCK:
+            if _BINDING is None:
+                path = os.path.join(LIB_DIR, "marathon_binding.so")
+                if not os.path.exists(path):
+                    raise RuntimeError(
+                        f"{path} is missing: build it with "
+                        "`python -c 'import __graft_entry__ as g; g.build()'`")
+                from importlib.machinery import ExtensionFileLoader
+                from importlib.util import module_from_spec, spec_from_loader
+
+                loader = ExtensionFileLoader("marathon_binding", path)
+                module = module_from_spec(spec_from_loader("marathon_binding", loader))
+                loader.exec_module(module)
+                module.bind(ctypes.cast(cdll.mkv_scatter_shifted, ctypes.c_void_p).value)
+                _BINDING = module
+    return _BINDING
 
 
 def check(rc: int) -> None:

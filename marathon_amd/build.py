@@ -1,8 +1,10 @@
-"""In-tree build of the HIP library (gfx950 only).
+"""In-tree build of the HIP library (gfx950 only) and of its CPython binding.
 
 ``python -m marathon_amd.build`` (or ``__graft_entry__.build()``) compiles
 ``csrc/kvshift.hip`` into ``_lib/libmarathon_kvshift.so`` with hipcc.  It always
 recompiles: the build is a few seconds and a stale library is worse than a slow one.
+:func:`build_binding` compiles ``csrc/binding.cpp``, the per-layer call's path from torch
+tensors, into ``_lib/marathon_binding.so`` with g++.
 :func:`build_test_libraries` compiles the GPU tests' own HIP helpers (``tests/hip``)
 into ``tests/_lib`` with the same flags.
 """
@@ -13,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -20,6 +23,8 @@ SRC = os.path.join(HERE, "csrc", "kvshift.hip")
 INCLUDE = os.path.join(ROOT, "include")
 OUT_DIR = os.path.join(HERE, "_lib")
 OUT = os.path.join(OUT_DIR, "libmarathon_kvshift.so")
+BINDING_SRC = os.path.join(HERE, "csrc", "binding.cpp")
+BINDING_OUT = os.path.join(OUT_DIR, "marathon_binding.so")
 TEST_SRC_DIR = os.path.join(ROOT, "tests", "hip")
 TEST_OUT_DIR = os.path.join(ROOT, "tests", "_lib")
 
@@ -91,6 +96,34 @@ def build_library(verbose: bool = False) -> str:
     return out
 
 
+def build_binding(verbose: bool = False) -> str:
+    """The CPython module over the installed torch's own headers and libraries."""
+    import torch
+
+    home = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    os.makedirs(OUT_DIR, exist_ok=True)
+    tmp = BINDING_OUT + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f"-I{INCLUDE}",
+           "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", os.path.join(home, "include"),
+           "-isystem", os.path.join(home, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), BINDING_SRC,
+           f"-L{os.path.join(home, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", f"-Wl,-rpath,{os.path.join(home, 'lib')}", "-o", tmp]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + res.stderr)
+    if verbose and res.stderr:
+        print(res.stderr, file=sys.stderr)
+    os.replace(tmp, BINDING_OUT)
+    return BINDING_OUT
+
+
 def _compile_c_host(src: str, out: str, verbose: bool) -> str:
     """A C host program against the library's C ABI and the HIP runtime, built by gcc
     (no HIP compiler involved: this is what an outside C caller does)."""
@@ -132,5 +165,6 @@ def build_test_libraries(verbose: bool = False) -> list:
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_binding(verbose=True))
     for path in build_test_libraries(verbose=True):
         print(path)

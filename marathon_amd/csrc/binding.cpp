@@ -3,9 +3,9 @@
 // scatter(src, kv, slots, block_size, hnd, shift, k_scale, error_flags) is
 // shift_kernels.scatter_shifted's usual call: it reads the tensors through torch's C++
 // interface, checks what that function checks and calls mkv_scatter_shifted on the current
-// stream.  Through Python methods and ctypes the same call spends 3.6 us of 6.7 around its
-// launch, which is longer than the kernel of a short span runs (2.4 us for 300 tokens), so
-// the caller's loop over layers is bound by it.
+// stream.  Through Python methods and ctypes the same call spent 3.6 us of its 6.7 around
+// the launch, longer than the kernel of a short span runs (2.4 us for 300 tokens), so a loop
+// over layers was bound by it: 28 calls of 301 fp16 tokens 168 -> 101 us.
 //
 // Returns the library's status, or None wherever the call is not the usual one (tensors
 // that need a copy or a conversion, subclasses and wrapped tensors, another current device,

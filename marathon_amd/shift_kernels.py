@@ -220,6 +220,15 @@ def _scale_tensor(k_scale, device) -> torch.Tensor:
     return t
 
 
+_usual_call = None  # the binding's scatter, once loaded
+
+
+def _load_usual_call():
+    global _usual_call
+    _usual_call = _lib.binding().scatter
+    return _usual_call
+
+
 def scatter_shifted(
     src: torch.Tensor,
     kv: torch.Tensor,
@@ -238,7 +247,17 @@ def scatter_shifted(
     delta 0) is a plain scatter (shift_kernels.py:166-179).  Asynchronous on the
     current stream.  ``k_scale`` (fp8 caches only) is the layer's K scale;
     ``error_flags`` an optional int32 device tensor that collects out-of-range bits.
+
+    A call whose tensors need no conversion goes through the CPython binding, which makes
+    the checks below on the tensors themselves; it answers None, with nothing launched,
+    for any other call.
     """
+    rc = (_usual_call or _load_usual_call())(src, kv, slots, block_size, hnd, shift, k_scale,
+                                             error_flags)
+    if rc is not None:
+        if rc:
+            _lib.check(rc)
+        return
     if not kv.is_cuda:
         raise RuntimeError(
             "scatter_shifted: kv is not on a HIP device; marathon_amd has no CPU path"
