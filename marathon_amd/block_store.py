@@ -87,6 +87,7 @@ class _BlockEntry(Window):
     held: int = 0  # pool blocks this session owns
     valid: list = field(default_factory=list)  # interval policy: sorted disjoint [lo, hi)
     layers: set = field(default_factory=set)  # layers saved at least once
+    saved_as: tuple = ()  # the last step's layers, all of them in `layers`
 
 
 def _add_interval(ivs: list, lo: int, hi: int) -> None:
@@ -132,6 +133,7 @@ class BlockShiftStore(StoreCore):
         self._plane_lists: dict[tuple, tuple] = {}  # layers -> (pools existing, (k, v))
         self._target_lists: dict[tuple, tuple] = {}  # layers -> (pools existing, pools)
         self._sig_ok: dict[tuple, tuple] = {}  # layers -> the row signature all pools have
+        self._freed = 0  # how often blocks went back to the pool
 
     # --------------------------------------------------------------- store hooks
 
@@ -194,6 +196,7 @@ class BlockShiftStore(StoreCore):
                 heapq.heappush(self._free, b)
             entry.held -= int(freed.size)
             part[:] = -1
+            self._freed += 1
         elif entry.table.size == 0 or entry.table[-1] >= 0:
             return  # nothing in the range and no unheld tail to trim (an append)
         live = np.flatnonzero(entry.table >= 0)
@@ -291,6 +294,22 @@ class BlockShiftStore(StoreCore):
         """Whether every position of ``[dst_start, dst_start + n)`` has a block."""
         return self._positions_ok(self._sessions.get(session), dst_start, n)
 
+    def _targets(self, layers, row_shape, dtype, device) -> tuple:
+        """``(key, pools)`` of ``layers`` for rows of this signature, made where missing;
+        ``key`` is one tuple object per distinct list of layers."""
+        sig = (tuple(row_shape), dtype)
+        key = tuple(layers)
+        hit = self._target_lists.get(key)
+        if hit is not None and hit[0] == len(self._pools) and self._sig_ok.get(key) == sig:
+            return hit[2], hit[1]  # the steady state: every pool exists with these rows
+        pools, sigs = self._pools, self._sigs
+        out = [pools[layer] if sigs.get(layer) == sig else
+               self._pool_for(layer, row_shape, dtype, device) for layer in layers]
+        key = key if hit is None else hit[2]
+        self._target_lists[key] = (len(self._pools), out, key)
+        self._sig_ok[key] = sig
+        return key, out
+
     def write_targets(
         self, session: str, layers, dst_start: int, n: int, row_shape, dtype, device
     ) -> list | None:
@@ -298,21 +317,56 @@ class BlockShiftStore(StoreCore):
         entry = self._sessions.get(session)
         if not self._positions_ok(entry, dst_start, n):
             return None
-        sig = (tuple(row_shape), dtype)
-        key = tuple(layers)
-        hit = self._target_lists.get(key)
-        if hit is not None and hit[0] == len(self._pools) and self._sig_ok.get(key) == sig:
-            out = hit[1]  # the steady state: every pool exists with these rows
-        else:
-            pools, sigs = self._pools, self._sigs
-            out = [pools[layer] if sigs.get(layer) == sig else
-                   self._pool_for(layer, row_shape, dtype, device) for layer in layers]
-            self._target_lists[key] = (len(self._pools), out)
-            self._sig_ok[key] = sig
+        key, out = self._targets(layers, row_shape, dtype, device)
         if not entry.layers.issuperset(key):
             entry.layers.update(key)
         self.saved_token_layers += n * len(out)
         return out
+
+    def take_saves(self, saves, layers, row_shape, dtype, device) -> list:
+        """:meth:`reserve` and :meth:`write_targets` of a step's saves in order, with the
+        same state, counters and LRU order after: those that hold blocks for all their
+        positions at the end, as ``(save, session record, n)``.
+
+        Most saves append to a session inside blocks it has (a decode step's does 15 times
+        in 16): such a one only moves its record's end and LRU place, which is all that
+        ``reserve`` would do, so it is done here; any other goes through ``reserve``."""
+        sessions, bs, budget = self._sessions, self.block_size, self.budget
+        append = self.truncate and self.allocate
+        freed, key, layers_n, taken = self._freed, None, 0, []
+        for save in saves:
+            n = save.n
+            if n == 0:
+                continue
+            session, start = save.session, save.dst_start
+            end = start + n
+            entry = sessions.get(session)
+            if (append and entry is not None and 0 <= entry.base and 0 <= start <= entry.filled
+                    and end <= budget
+                    and entry.table.size == (last := (end - 1) // bs) + 1
+                    and entry.table[last] >= 0
+                    and (start // bs == last or bool((entry.table[start // bs:last] >= 0).all()))):
+                sessions.move_to_end(session)
+                entry.filled = end
+            else:
+                if not self.reserve(session, start, n):
+                    continue
+                entry = sessions[session]
+                if not self._positions_ok(entry, start, n):
+                    continue
+            if key is None:
+                key, pools = self._targets(layers, row_shape, dtype, device)
+                layers_n = len(pools)
+            if entry.saved_as is not key:
+                entry.layers.update(key)
+                entry.saved_as = key
+            self.saved_token_layers += n * layers_n
+            taken.append((save, entry, n))
+        if self._freed != freed and len(taken) > 1:
+            # a later save may have truncated or evicted what an earlier one was given
+            taken = [(sv, sessions[sv.session], n) for sv, _, n in taken
+                     if self.holds_blocks(sv.session, sv.dst_start, n)]
+        return taken
 
     def write_target(
         self, session: str, layer: str, dst_start: int, n: int, row_shape, dtype, device

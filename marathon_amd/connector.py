@@ -225,6 +225,21 @@ def table_window(table: np.ndarray, pos: int, n: int, block_size: int):
     return table[k0:k1], pos - k0 * block_size
 
 
+def _windows(spans, block_size: int) -> tuple:
+    """The :func:`table_window` of each ``(table, pos, n)``: the windows concatenated, and
+    per item ``(pos, offset)`` (``pos`` within its window, which starts at ``offset``)."""
+    tabs, rows, off = [], [], 0
+    for table, pos, n in spans:
+        k0 = pos // block_size
+        k1 = -(-(pos + n) // block_size)
+        if pos < 0 or k1 > table.size:
+            table_window(table, pos, n, block_size)  # raises
+        tabs.append(table[k0:k1])
+        rows.append((pos - k0 * block_size, off))
+        off += k1 - k0
+    return tabs[0] if len(tabs) == 1 else np.concatenate(tabs), rows
+
+
 def paged_index(items: list, block_size: int):
     """Address the paged side of a batch of loads or saves: ``(mode, index, rows)``.
 
@@ -234,18 +249,18 @@ def paged_index(items: list, block_size: int):
     the device.  Otherwise the slots are concatenated (int64; ``from_blocks`` items are
     expanded on the host) and each item gets ``(0, offset)`` into them.
     """
-    if all(it.slots is None for it in items):
-        tabs, rows, off = [], [], 0
+    if all([it.slots is None for it in items]):
+        spans = []
         tables: dict[int, np.ndarray] = {}  # items of one request share its block table
         for it in items:
-            t = tables.get(id(it.block_ids))
-            if t is None:
-                t = tables[id(it.block_ids)] = _int32_table(it.block_ids)
-            win, pos = table_window(t, it.paged_pos, it.n, block_size)
-            tabs.append(win)
-            rows.append((pos, off))
-            off += win.size
-        return "table", tabs[0] if len(tabs) == 1 else np.concatenate(tabs), rows
+            t = it.block_ids
+            if type(t) is not np.ndarray or t.dtype != np.int32 or t.ndim != 1:
+                ids = t
+                t = tables.get(id(ids))
+                if t is None:
+                    t = tables[id(ids)] = _int32_table(ids)
+            spans.append((t, int(it.dst_start), max(int(it.n_tokens), 0)))
+        return ("table", *_windows(spans, block_size))
     parts, rows, off = [], [], 0
     for it in items:
         if it.slots is None:
@@ -256,18 +271,6 @@ def paged_index(items: list, block_size: int):
         rows.append((0, off))
         off += int(sl.numel())
     return "slots", torch.cat(parts), rows
-
-
-def _store_windows(store, items, start_of) -> tuple:
-    """The block store's side of a batch: each item's window of its session's block
-    table, concatenated, and per item ``(pos, offset)`` (see :func:`table_window`)."""
-    tabs, rows, off = [], [], 0
-    for it in items:
-        win, pos = table_window(store.table(it.session), start_of(it), it.n, store.block_size)
-        tabs.append(win)
-        rows.append((pos, off))
-        off += win.size
-    return tabs[0] if len(tabs) == 1 else np.concatenate(tabs), rows
 
 
 def detect_hnd(shape, block_size: int) -> bool:
@@ -354,7 +357,7 @@ class ShiftLoader:
         self.last_plan: ShiftPlan | SmallShifts | None = None
         self._sets = _CacheSets(self.block_size)
         self._small = _SmallRunners()
-        self._k_scale_key: tuple | None = None
+        self._k_scale_key: list | None = None
         self._k_scale_t: torch.Tensor | None = None
 
     @property
@@ -419,7 +422,9 @@ class ShiftLoader:
             src = self._sets.get("store", [caches], "nhd", self.store.block_size,
                                  v_caches=None if v_caches is None else [v_caches])
             src_mode = "table"
-            src_index, src_rows = _store_windows(self.store, taken, lambda ld: ld.src_start)
+            src_index, src_rows = _windows(
+                [(self.store.table(ld.session), ld.src_start, ld.n) for ld in taken],
+                self.store.block_size)
             for load, (spos, sidx), (dpos, didx) in zip(taken, src_rows, dst_rows):
                 rows.append((spos, dpos, sidx, didx, load.n, int(load.delta), 0, 0))
         else:
@@ -441,7 +446,7 @@ class ShiftLoader:
             t0 = time.perf_counter()
         small = self._small.get(src, dst, src_mode, dst_mode, self.inv_freq, k_scale)
         if small.fits(len(rows), tokens):  # a short load: no plan to build
-            small.run(rows, _host(src_index), _host(dst_index))
+            small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)
             plan = small
         else:
             plan = ShiftPlan(
@@ -485,9 +490,11 @@ class ShiftLoader:
     def _k_scale(self, names) -> torch.Tensor:
         """The layers' K scales as one fp32 CPU tensor, rebuilt only when a scale changed
         (``k_scales`` is shared with the saver and may fill in later)."""
-        key = tuple(float(self.k_scales.get(name, 1.0)) for name in names)
+        get = self.k_scales.get
+        key = [float(get(name, 1.0)) for name in names]
         if self._k_scale_key != key:
-            self._k_scale_key, self._k_scale_t = key, torch.tensor(key, dtype=torch.float32)
+            self._k_scale_key = key
+            self._k_scale_t = torch.tensor(key, dtype=torch.float32)
         return self._k_scale_t
 
     def _verify(self, name: str, load: Load, k_scale, layer: int) -> None:
@@ -715,6 +722,7 @@ class ShiftSaver:
         self.last_plan: ShiftPlan | None = None
         self._sets = _CacheSets(self.block_size)
         self._pending: list = []  # deferred: (layer name, paged cache, the step's saves)
+        self.record = self._pending.append  # such a triple, for the next wait_for_save
         self._geo: dict[tuple, tuple] = {}  # the caches of a step -> their geometry
         self._small = _SmallRunners()
 
@@ -742,7 +750,8 @@ class ShiftSaver:
 
     def _plan(self, names: list, caches: list, saves: list) -> int:
         row_shape, dtype, device, paged = self._geometry(caches)
-        blocky = isinstance(self.store, BlockShiftStore)
+        if isinstance(self.store, BlockShiftStore):
+            return self._plan_blocks(names, saves, row_shape, dtype, device, paged)
         groups: dict[str, int] = {}
         bufs: list[list] = []
         taken = []
@@ -764,30 +773,36 @@ class ShiftSaver:
             else:
                 bufs[g] = targets  # a save may have grown (reallocated) the buffers
             taken.append(save)
-        if blocky and len(taken) > 1:
-            # a later save of the same call may have truncated an earlier one's blocks
-            taken = [sv for sv in taken if self.store.holds_blocks(sv.session, sv.dst_start, sv.n)]
         if not taken:
             return 0
         src_mode, src_index, src_rows = paged_index(taken, self.block_size)
         rows = []
-        if blocky:
-            caches, v_caches = self.store.kernel_views(names)
-            dst = self._sets.get("store", [caches], "nhd", self.store.block_size,
-                                 v_caches=None if v_caches is None else [v_caches])
-            dst_mode = "table"
-            dst_index, dst_rows = _store_windows(self.store, taken, lambda sv: sv.dst_start)
-            for sv, (spos, sidx), (dpos, didx) in zip(taken, src_rows, dst_rows):
-                rows.append((spos, dpos, sidx, didx, sv.n, 0, 0, 0))
-        else:
-            dst = self._sets.get("store", bufs, "flat")
-            dst_mode, dst_index = "flat", None
-            for sv, (spos, sidx) in zip(taken, src_rows):
-                rows.append((spos, int(sv.dst_start), sidx, 0, sv.n, 0, 0, groups[sv.session]))
-        tokens = sum(sv.n for sv in taken)
+        dst = self._sets.get("store", bufs, "flat")
+        for sv, (spos, sidx) in zip(taken, src_rows):
+            rows.append((spos, int(sv.dst_start), sidx, 0, sv.n, 0, 0, groups[sv.session]))
+        return self._launch(names, paged, dst, rows, src_mode, src_index, "flat", None)
+
+    def _plan_blocks(self, names: list, saves: list, row_shape, dtype, device, paged) -> int:
+        store = self.store
+        taken = store.take_saves(saves, names, row_shape, dtype, device)
+        if not taken:
+            return 0
+        caches, v_caches = store.kernel_views(names)
+        dst = self._sets.get("store", [caches], "nhd", store.block_size,
+                             v_caches=None if v_caches is None else [v_caches])
+        src_mode, src_index, src_rows = paged_index([t[0] for t in taken], self.block_size)
+        dst_index, dst_rows = _windows(
+            [(entry.table, sv.dst_start, n) for sv, entry, n in taken], store.block_size)
+        rows = [(spos, dpos, sidx, didx, n, 0, 0, 0)
+                for (_, _, n), (spos, sidx), (dpos, didx) in zip(taken, src_rows, dst_rows)]
+        return self._launch(names, paged, dst, rows, src_mode, src_index, "table", dst_index)
+
+    def _launch(self, names: list, paged, dst, rows: list, src_mode, src_index, dst_mode,
+                dst_index) -> int:
+        tokens = sum([r[4] for r in rows])
         small = self._small.get(paged, dst, src_mode, dst_mode, None)
         if small.fits(len(rows), tokens):  # a decode step: no plan to build
-            small.run(rows, _host(src_index), _host(dst_index))
+            small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)
             self.last_plan = small
             return tokens * len(names)
         plan = ShiftPlan(
@@ -814,14 +829,21 @@ class ShiftSaver:
         step is final, and the store ends the step in the state per-layer saves leave.
         """
         if self.deferred:
-            self._pending.append((layer_name, kv_layer, saves))
+            self.record((layer_name, kv_layer, saves))
             return 0
         return self._plan([layer_name], [kv_layer], saves)
 
     def wait_for_save(self) -> int:
         """Flush the deferred layers: one launch per distinct list of saves (a step has
         one).  Returns the token-layers saved; 0 when nothing is pending."""
-        pending, self._pending = self._pending, []
+        pending = self._pending[:]
+        self._pending.clear()
+        if not pending:
+            return 0
+        saves = pending[0][2]
+        if all([item[2] is saves for item in pending]):
+            names, caches, _ = zip(*pending)
+            return self._plan(names, caches, saves)
         groups: dict[int, tuple] = {}
         for name, cache, saves in pending:
             names, caches, _ = groups.setdefault(id(saves), ([], [], saves))

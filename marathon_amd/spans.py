@@ -21,7 +21,10 @@ or the one shared paged cache.
 from __future__ import annotations
 
 import ctypes
+import functools
+import struct
 from dataclasses import dataclass
+from itertools import chain
 
 import numpy as np
 import torch
@@ -567,6 +570,13 @@ class ShiftPlan:
             _lib.check(L.mkv_shift_spans(ctypes.byref(d), ctypes.c_void_p(stream)))
 
 
+@functools.lru_cache(maxsize=128)
+def _span_struct(n: int) -> struct.Struct:
+    """``n`` span rows (``mkv_span_t``) from their fields: half the time of assigning the
+    tuples to a structured array."""
+    return struct.Struct("<" + "4q4i" * n)
+
+
 class SmallShifts:
     """Shifts with no :class:`ShiftPlan` to build: the steady state of a serving loop (a
     decode step's saves, a prefill chunk's save, a step's loads).
@@ -656,9 +666,10 @@ class SmallShifts:
         return 0 < n_spans <= _lib.MKV_MAX_SPANS and tokens > 0
 
     def run(self, rows: list, src_index: np.ndarray | None, dst_index: np.ndarray | None,
-            error_flags: torch.Tensor | None = None) -> None:
+            error_flags: torch.Tensor | None = None, tokens: int | None = None) -> None:
         """Shift ``rows`` (``mkv_span_t`` field tuples) on the current stream, their
-        source and destination indices given as host arrays (None for ``flat``).
+        source and destination indices given as host arrays (None for ``flat``);
+        ``tokens``: the sum of the rows' positive token counts, where the caller has it.
 
         Up to ``MKV_SMALL_MAX_SPANS`` spans and ``MKV_SMALL_MAX_INDEX`` index entries a
         side, the rows and windows travel in the launch itself
@@ -666,7 +677,8 @@ class SmallShifts:
         n = len(rows)
         n_src = 0 if src_index is None else src_index.size
         n_dst = 0 if dst_index is None else dst_index.size
-        tokens = sum(max(int(r[4]), 0) for r in rows)
+        if tokens is None:
+            tokens = sum(max(int(r[4]), 0) for r in rows)
         if (self.eligible_geometry and n <= _lib.MKV_SMALL_MAX_SPANS
                 and n_src <= _lib.MKV_SMALL_MAX_INDEX and n_dst <= _lib.MKV_SMALL_MAX_INDEX
                 and tokens * self.dst.layers <= SMALL_ARGS_MAX_TOKEN_LAYERS):
@@ -692,13 +704,14 @@ class SmallShifts:
         self.tokens = tokens
         # mkv_shift_workspace_size: the spans' tables, then 32 bytes a token
         size = (n * 8 * self.rotary + 255) // 256 * 256 + 32 * tokens
-        rows = np.array(rows, dtype=_lib.SPAN_DTYPE)
+        spans = np.empty(n, dtype=_lib.SPAN_DTYPE)
+        _span_struct(n).pack_into(spans.view(np.uint8), 0, *chain.from_iterable(rows))
         if size <= HOST_PLAN_MAX_BYTES:
-            raised = self._plan_here(rows, src_index, dst_index, tokens, size)
+            raised = self._plan_here(spans, src_index, dst_index, tokens, size)
             if raised and error_flags is not None:
                 error_flags.bitwise_or_(raised)
         else:
-            self._stage(rows, src_index, dst_index, tokens, size)
+            self._stage(spans, src_index, dst_index, tokens, size)
         self.launch(error_flags=error_flags)
 
     def _upload(self, host: torch.Tensor) -> int:

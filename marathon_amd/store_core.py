@@ -126,12 +126,14 @@ class StoreCore:
     def _evict_until(self, session: str, fits) -> bool:
         """Drop whole sessions other than ``session``, least recently used first, until
         ``fits()``; returns whether it fits in the end."""
+        if fits():
+            return True
         for victim in [s for s in self._sessions if s != session]:
-            if fits():
-                return True
             self.drop(victim)
             self.evictions += 1
-        return fits()
+            if fits():
+                return True
+        return False
 
     def reserve(self, session: str, dst_start: int, n: int) -> bool:
         """Make room for positions ``[dst_start, dst_start + n)`` of ``session``.

@@ -278,9 +278,8 @@ class MarathonShiftConnector(_ConnectorBase):
         """Record the layer; the step's saves run in ``wait_for_save``
         (vllm_shift_connector.py:539-553)."""
         meta = self._get_connector_metadata()
-        if meta is None or not meta.saves:
-            return
-        self._saver.save_kv_layer(layer_name, kv_layer, meta.saves)
+        if meta is not None and meta.saves:
+            self._saver.record((layer_name, kv_layer, meta.saves))
 
     def wait_for_save(self) -> None:
         """Save every layer recorded this step in one launch."""
