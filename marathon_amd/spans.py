@@ -43,6 +43,15 @@ MODES = {"flat": _lib.MKV_ADDR_FLAT, "slots": _lib.MKV_ADDR_SLOTS, "table": _lib
 #: then slot) before it can load its data, where a record from the plan pass carries the
 #: token's rows.  Above 2,560 rows the direct kernel moves four layers per workgroup.
 DIRECT_MAX_TOKEN_LAYERS = 20480
+#: The most bytes of K and V such a shift may read, by element size (default the last):
+#: resolving a token again for each of its layers costs a direct workgroup the more, the
+#: more workgroups a token and layer take and the fewer bytes each moves.  Kept plans of 2
+#: spans x 40 layers, us a launch, direct / two launches: fp8 8 heads of 128, 150 tokens (12
+#: MB) 9.9 / 11.2, 200 (16 MB) 13.0 / 12.1, 511 24.8 / 21.1; 16 heads, 64 tokens (10 MB) 9.4
+#: / 10.7, 100 (16 MB) 14.1 / 12.2, 511 46.2 / 37.2; bf16 16 heads, 303 tokens (99 MB) 37.7
+#: / 39.6, 400 (131 MB) 50.6 / 49.2, 511 64.9 / 59.9; fp32 8 heads, 511 tokens (167 MB) 61.9
+#: / 58.7.
+DIRECT_MAX_BYTES = {1: 14 << 20, None: 120 << 20}
 #: SmallShifts puts a step's spans and index windows in the launch's own arguments up to
 #: this many (token, layer) rows: that saves the host its staging copy, but every
 #: workgroup then reads the arguments, which costs more than the copy from about 64
@@ -288,7 +297,8 @@ class ShiftPlan:
     uploaded once per :class:`CacheSet`.
 
     ``direct``: None (default) takes the library's single-launch path up to
-    :data:`DIRECT_MAX_TOKEN_LAYERS` rows whenever :meth:`direct_eligible` allows it,
+    :data:`DIRECT_MAX_TOKEN_LAYERS` rows and :data:`DIRECT_MAX_BYTES` whenever
+    :meth:`direct_eligible` allows it,
     with the token prefix and the per-span rotation tables computed here
     (:func:`span_tables`); False always runs the two-launch path (plan pass and
     workspace), True asks for the direct path where eligible.
@@ -376,7 +386,9 @@ class ShiftPlan:
         # the direct path (one launch, no workspace) for small shifts, where the plan
         # pass's launch dominates; the token prefix and per-span tables come from here
         if direct is None:
-            direct = self.tokens * dst.layers <= DIRECT_MAX_TOKEN_LAYERS
+            most = DIRECT_MAX_BYTES.get(dst.first.element_size(), DIRECT_MAX_BYTES[None])
+            direct = (self.tokens * dst.layers <= DIRECT_MAX_TOKEN_LAYERS
+                      and self.algorithmic_bytes // 2 <= most)
         self.direct = bool(direct) and self.direct_eligible(src, dst, self.n_spans)
         starts_off = tables_off = None
         if self.direct:
