@@ -1,0 +1,31 @@
+"""The CPython binding as built, on the CPU: it has no thread-local storage (a TLS block that
+a thread has not touched slows every other library's TLS access in it), and it leaves calls
+on anything but GPU tensors to the general path."""
+
+from __future__ import annotations
+
+import os
+import struct
+
+import torch
+
+from marathon_amd import _lib
+
+PT_TLS = 7
+
+
+def test_binding_has_no_tls_segment():
+    with open(os.path.join(_lib.LIB_DIR, "marathon_binding.so"), "rb") as f:
+        elf = f.read()
+    assert elf[:5] == b"\x7fELF\x02"
+    at, = struct.unpack_from("<Q", elf, 32)  # e_phoff
+    size, count = struct.unpack_from("<HH", elf, 54)  # e_phentsize, e_phnum
+    assert PT_TLS not in [struct.unpack_from("<I", elf, at + k * size)[0] for k in range(count)]
+
+
+def test_binding_leaves_other_calls():
+    scatter = _lib.binding().scatter
+    src, kv = torch.zeros(2, 8, 128), torch.zeros(4, 8, 16, 128)
+    slots = torch.zeros(2, dtype=torch.int64)
+    assert scatter(src, kv, slots, 16, True, None, None, None) is None
+    assert scatter(None, 3, "x", 16, True, None, None, None) is None
