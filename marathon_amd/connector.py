@@ -206,6 +206,11 @@ def _host(index) -> np.ndarray | None:
     return index.numpy()
 
 
+def _on_device(index) -> bool:
+    """Whether a step's index is on the GPU: a plan reads it there, in place."""
+    return isinstance(index, torch.Tensor) and index.is_cuda
+
+
 def _int32_table(t) -> np.ndarray:
     if isinstance(t, np.ndarray) and t.dtype == np.int32:
         return t.reshape(-1)
@@ -444,8 +449,9 @@ class ShiftLoader:
         if self.timing:
             torch.cuda.synchronize(dst.first.device)
             t0 = time.perf_counter()
-        small = self._small.get(src, dst, src_mode, dst_mode, self.inv_freq, k_scale)
-        if small.fits(len(rows), tokens):  # a short load: no plan to build
+        small = None if _on_device(dst_index) else self._small.get(
+            src, dst, src_mode, dst_mode, self.inv_freq, k_scale)
+        if small is not None and small.fits(len(rows), tokens):  # no plan to build
             small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)
             plan = small
         else:
@@ -719,7 +725,7 @@ class ShiftSaver:
         self.store = store
         self.block_size = int(block_size)
         self.deferred = bool(deferred)
-        self.last_plan: ShiftPlan | None = None
+        self.last_plan: ShiftPlan | SmallShifts | None = None
         self._sets = _CacheSets(self.block_size)
         self._pending: list = []  # deferred: (layer name, paged cache, the step's saves)
         self.record = self._pending.append  # such a triple, for the next wait_for_save
@@ -800,8 +806,9 @@ class ShiftSaver:
     def _launch(self, names: list, paged, dst, rows: list, src_mode, src_index, dst_mode,
                 dst_index) -> int:
         tokens = sum([r[4] for r in rows])
-        small = self._small.get(paged, dst, src_mode, dst_mode, None)
-        if small.fits(len(rows), tokens):  # a decode step: no plan to build
+        small = None if _on_device(src_index) else self._small.get(
+            paged, dst, src_mode, dst_mode, None)
+        if small is not None and small.fits(len(rows), tokens):  # no plan to build
             small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)
             self.last_plan = small
             return tokens * len(names)
