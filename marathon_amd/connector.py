@@ -737,7 +737,8 @@ class ShiftSaver:
         out once per distinct tuple of cache tensors (vLLM passes the same ones every
         step)."""
         # keyed by the tensors' ids (a tuple of tensors would hash each tensor through
-        # Python); the entry's CacheSet holds the tensors, so no id is reused meanwhile
+        # Python); the entry holds the tensors, so no id is reused meanwhile (its CacheSet
+        # alone does not: of split caches it has views, which need not keep their base)
         key = tuple(map(id, caches))
         hit = self._geo.get(key)
         if hit is None:
@@ -751,8 +752,8 @@ class ShiftSaver:
                              v_caches=[[v for _, _, v in planes]] if split else None)
             if len(self._geo) >= 64:  # caches replaced many times over
                 self._geo.clear()
-            hit = self._geo[key] = (row_shape, first.dtype, first.device, paged)
-        return hit
+            hit = self._geo[key] = (row_shape, first.dtype, first.device, paged, tuple(caches))
+        return hit[:4]
 
     def _plan(self, names: list, caches: list, saves: list) -> int:
         row_shape, dtype, device, paged = self._geometry(caches)
