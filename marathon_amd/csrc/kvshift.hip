@@ -2351,7 +2351,8 @@ int shift_spans(const mkv_shift_desc_t* d, void* stream, PlanFrom from) {
     }
     const size_t lds = sizeof(int64_t) * (static_cast<size_t>(d->n_spans) + 1);
     pp.rec_groups = static_cast<int32_t>(plan_grid);  // the order kernel's groups too
-    const bool few = !ordered && d->n_spans <= kFewSpans &&
+    // plan_few_kernel makes tables only in workgroups past rec_groups
+    const bool few = MKV_PLAN_TABLE_GROUPS && !ordered && d->n_spans <= kFewSpans &&
                      pp.src.bs_shift >= 0 && pp.dst.bs_shift >= 0;
     hipLaunchKernelGGL(few ? plan_few_kernel : plan_kernel,
                        dim3(static_cast<unsigned>(plan_grid + tab_grid)), dim3(kPlanThreads),
