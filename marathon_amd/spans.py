@@ -283,6 +283,33 @@ class _Staging:
         return host.to(device, non_blocking=True)
 
 
+class _Uploads:
+    """The copies that a shift's launches read -- ``own``, made on the current stream, and
+    its cache sets' base-address tables, each made where its set was first used -- and the
+    streams whose launches are ordered after all of them (``synced``)."""
+
+    def __init__(self, device, sets, own: list) -> None:
+        self.device = device
+        self.stream = current_stream(device)
+        self.own = own
+        self.ready = [cs.device_tables(device)[3] for cs in sets]
+        self.synced = {self.stream} if all(
+            cs.upload_stream == self.stream for cs in sets) else set()
+
+    def order(self, stream: int, more=()) -> None:
+        """Before a launch on a stream that is not in ``synced``: it waits for the copies
+        and keeps them (and ``more``) alive.  A stream that is being captured cannot wait
+        for them, so it is asked again at its next launch."""
+        ext = torch.cuda.ExternalStream(stream, device=self.device)
+        for t in (*self.own, *more):
+            t.record_stream(ext)
+        if not torch.cuda.is_current_stream_capturing():
+            ext.wait_stream(torch.cuda.ExternalStream(self.stream, device=self.device))
+            for ready in self.ready:
+                ext.wait_event(ready)
+            self.synced.add(stream)
+
+
 class ShiftPlan:
     """A batched shift, resident on the device and launchable any number of times.
 
@@ -427,17 +454,12 @@ class ShiftPlan:
         on_device = self.device.index == torch.cuda.current_device()
         with _on(self.device, on_device):
             # the caches' base-address tables: uploaded once per CacheSet
-            self._tables_ready = []
-            sides = []
-            for cs in (src, dst):
-                k_ptr, v_ptr, caps_ptr, ready, _ = cs.device_tables(self.device)
-                self._tables_ready.append(ready)
-                sides.append((k_ptr, v_ptr, caps_ptr))
+            sides = [cs.device_tables(self.device)[:3] for cs in (src, dst)]
             # this plan's own arrays: one stream-ordered copy on the current stream
             blob = stage.upload(self.device)
-            self._build_stream = current_stream(self.device)
-        self._keep.append(blob)
-        self._synced = {self._build_stream}
+            self._keep.append(blob)
+            self._uploads = _Uploads(self.device, (src, dst), self._keep)
+        self._uploads.synced.add(self._uploads.stream)
         base = blob.data_ptr()
 
         def ptr(item) -> int | None:
@@ -564,18 +586,8 @@ class ShiftPlan:
 
     def _launch(self, stream: int, error_flags: torch.Tensor | None) -> None:
         L = _lib.lib()
-        if stream not in self._synced:
-            # the plan's arrays were copied on the stream current at build time, the
-            # caches' base-address tables when each set was first used
-            ext = torch.cuda.ExternalStream(stream, device=self.device)
-            if not torch.cuda.is_current_stream_capturing():
-                ext.wait_stream(torch.cuda.ExternalStream(self._build_stream,
-                                                          device=self.device))
-                for ready in self._tables_ready:
-                    ext.wait_event(ready)
-            for t in self._keep + ([] if self.workspace is None else [self.workspace]):
-                t.record_stream(ext)
-            self._synced.add(stream)
+        if stream not in self._uploads.synced:
+            self._uploads.order(stream, [] if self.workspace is None else [self.workspace])
         flags = error_flags.data_ptr() if error_flags is not None else None
         for d in self.descs:
             d.error_flags = flags
@@ -642,13 +654,8 @@ class SmallShifts:
                 scale_off = static.add(scale)
             blob = static.upload(self.device)
             self._keep.append(blob)
-            tables = [cs.device_tables(self.device) for cs in (src, dst)]
-            self._build_stream = current_stream(self.device)
-        sides = [t[:3] for t in tables]
-        self._ready = [t[3] for t in tables]
-        # streams that need not wait for these uploads
-        self._synced = {self._build_stream} if all(
-            cs.upload_stream == self._build_stream for cs in (src, dst)) else set()
+            sides = [cs.device_tables(self.device)[:3] for cs in (src, dst)]
+            self._uploads = _Uploads(self.device, (src, dst), self._keep)
         base = blob.data_ptr()
         d = self.desc = _lib.ShiftDesc()
         d.inv_freq = None if inv_off is None else base + inv_off
@@ -786,8 +793,8 @@ class SmallShifts:
         if stream is None:
             stream = current_stream(self.device)
         stream = int(stream)
-        if stream not in self._synced:
-            self._sync(stream)
+        if stream not in self._uploads.synced:
+            self._uploads.order(stream)
         L = _lib.lib()
         if self._last:
             d, fn = self.small_desc, L.mkv_shift_spans_small
@@ -797,18 +804,6 @@ class SmallShifts:
             d, fn = self._now, L.mkv_shift_spans
         d.error_flags = None if error_flags is None else error_flags.data_ptr()
         _lib.check(fn(ctypes.byref(d), stream))
-
-    def _sync(self, stream: int) -> None:
-        """A stream's first launch waits for what other streams uploaded: the caches'
-        base-address tables and this runner's frequencies and scales."""
-        ext = torch.cuda.ExternalStream(stream, device=self.device)
-        if not torch.cuda.is_current_stream_capturing():
-            ext.wait_stream(torch.cuda.ExternalStream(self._build_stream, device=self.device))
-            for ready in self._ready:
-                ext.wait_event(ready)
-        for t in self._keep:
-            t.record_stream(ext)
-        self._synced.add(stream)
 
     @property
     def algorithmic_bytes(self) -> int:
