@@ -459,7 +459,6 @@ class ShiftPlan:
             blob = stage.upload(self.device)
             self._keep.append(blob)
             self._uploads = _Uploads(self.device, (src, dst), self._keep)
-        self._uploads.synced.add(self._uploads.stream)
         base = blob.data_ptr()
 
         def ptr(item) -> int | None:

@@ -63,3 +63,33 @@ def test_a_captured_launch_does_not_count_as_ordered(streams):
     up.order(OTHER)
     assert LOG == [(OTHER, "stream", BUILD), (OTHER, "event", "src"), (OTHER, "event", "dst")]
     assert up.synced == {BUILD, OTHER}
+
+
+def test_a_plan_waits_for_tables_another_stream_uploaded(streams, monkeypatch):
+    """A plan built on one stream over cache sets whose base addresses went up on another:
+    its launches on the build stream wait for those."""
+    monkeypatch.setattr(spans._Staging, "upload",
+                        lambda self, device: torch.zeros(max(self.size, 256), dtype=torch.uint8))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)  # the CPU's index
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, s: None)
+    launched = []
+
+    class Lib:
+        def mkv_shift_spans(self, desc, stream):
+            launched.append(stream.value)
+            LOG.append("launch")
+            return 0
+
+    caches = [torch.zeros(32, 8, 128, dtype=torch.bfloat16) for _ in range(2)]
+    sets = [spans.CacheSet([[t]], "flat") for t in caches]
+    for cs, at in zip(sets, (BUILD, OTHER)):
+        cs.upload_stream = at
+        monkeypatch.setattr(cs, "device_tables", lambda device, at=at: (1, 2, None, at, caches[0]))
+    plan = spans.ShiftPlan(spans.span_array([(0, 0, 0, 0, 5, 0, 0, 0)]), *sets, inv_freq=None,
+                           dst_mode="flat", direct=True)
+    monkeypatch.setattr(spans._lib, "lib", Lib)
+    plan.launch()
+    assert launched == [BUILD] and (BUILD, "event", OTHER) in LOG[:LOG.index("launch")]
+    LOG.clear()
+    plan.launch()  # ordered once
+    assert LOG == ["launch"]
