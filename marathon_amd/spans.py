@@ -291,8 +291,9 @@ class _Uploads:
     def __init__(self, device, sets, own: list) -> None:
         self.device = device
         self.stream = current_stream(device)
-        self.own = own
-        self.ready = [cs.device_tables(device)[3] for cs in sets]
+        tables = [cs.device_tables(device) for cs in sets]
+        self.keep = [*own, *(t[4] for t in tables)]
+        self.ready = [t[3] for t in tables]
         self.synced = {self.stream} if all(
             cs.upload_stream == self.stream for cs in sets) else set()
 
@@ -301,7 +302,7 @@ class _Uploads:
         and keeps them (and ``more``) alive.  A stream that is being captured cannot wait
         for them, so it is asked again at its next launch."""
         ext = torch.cuda.ExternalStream(stream, device=self.device)
-        for t in (*self.own, *more):
+        for t in (*self.keep, *more):
             t.record_stream(ext)
         if not torch.cuda.is_current_stream_capturing():
             ext.wait_stream(torch.cuda.ExternalStream(self.stream, device=self.device))

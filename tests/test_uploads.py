@@ -93,3 +93,16 @@ def test_a_plan_waits_for_tables_another_stream_uploaded(streams, monkeypatch):
     LOG.clear()
     plan.launch()  # ordered once
     assert LOG == ["launch"]
+
+
+def test_base_tables_live_as_long_as_launches_on_other_streams(streams):
+    """The tables belong to the stream that uploaded them: freed there, their memory is
+    handed on in that stream's order, so every other stream that launches is recorded."""
+    own = [FakeTensor()]
+    sets = (FakeSet("src", BUILD), FakeSet("dst", THIRD))
+    up = spans._Uploads("dev", sets, own)
+    for stream in (BUILD, OTHER):
+        assert stream not in up.synced
+        up.order(stream)
+    assert [cs.blob.streams for cs in sets] == [{BUILD, OTHER}] * 2
+    assert up.synced == {BUILD, OTHER}
