@@ -639,7 +639,9 @@ class SmallShifts:
                         self._h_index[1].ctypes.data)
         self._flags = np.zeros(1, np.int32)  # mkv_plan_host's
         self._flags_at = self._flags.ctypes.data
-        self.buf = self.workspace = None  # the last step's, on the device
+        # the last step's, on the device: its plan, or its spans and indices and their plan
+        self.planned = self.staged = self.workspace = None
+        self._raised = 0  # the flags of the last step's plan, made on the host
         self._keep = []
         with _on(self.device, self.device.index == torch.cuda.current_device()):
             static = _Staging()
@@ -725,24 +727,25 @@ class SmallShifts:
         size = (n * 8 * self.rotary + 255) // 256 * 256 + 32 * tokens
         spans = np.empty(n, dtype=_lib.SPAN_DTYPE)
         _span_struct(n).pack_into(spans.view(np.uint8), 0, *chain.from_iterable(rows))
+        self._raised = 0
         if size <= HOST_PLAN_MAX_BYTES:
-            raised = self._plan_here(spans, src_index, dst_index, tokens, size)
-            if raised and error_flags is not None:
-                error_flags.bitwise_or_(raised)
-        else:
+            self._plan_here(spans, src_index, dst_index, tokens, size)
+        if size > HOST_PLAN_MAX_BYTES or self._raised:
             self._stage(spans, src_index, dst_index, tokens, size)
+        self._now = self.desc if size <= HOST_PLAN_MAX_BYTES else self.stage_desc
         self.launch(error_flags=error_flags)
 
-    def _upload(self, host: torch.Tensor) -> int:
+    def _upload(self, host: torch.Tensor) -> torch.Tensor:
         """A pinned buffer's copy on the device, in a buffer of this step's own (the
         allocator hands it on in stream order)."""
-        self.buf = torch.empty(host.numel(), dtype=torch.uint8, device=self.device)
-        self.buf.copy_(host, non_blocking=True)
-        return self.buf.data_ptr()
+        buf = torch.empty(host.numel(), dtype=torch.uint8, device=self.device)
+        return buf.copy_(host, non_blocking=True)
 
     def _plan_here(self, spans: np.ndarray, src_index, dst_index, tokens: int,
-                   size: int) -> int:
-        """Plan the step on the host; returns the flags of rows that will not be moved."""
+                   size: int) -> None:
+        """Plan the step on the host.  The plan holds no rows that cannot be moved, so it
+        raises no flags when launched: such a step is staged as well, for launches that
+        ask for them."""
         h = self.plan_desc
         h.spans, h.n_spans, h.total_tokens = spans.ctypes.data, spans.size, tokens
         windows = []  # alive until the call has read them
@@ -757,10 +760,11 @@ class SmallShifts:
         host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
         h.workspace, h.workspace_bytes = host.data_ptr(), size
         _lib.check(_lib.lib().mkv_plan_host(ctypes.byref(h), self._flags_at))
-        d = self._now = self.desc
+        self._raised = int(self._flags[0])
+        self.planned = self._upload(host)
+        d = self.desc
         d.n_spans, d.total_tokens = spans.size, tokens
-        d.workspace, d.workspace_bytes = self._upload(host), size
-        return int(self._flags[0])
+        d.workspace, d.workspace_bytes = self.planned.data_ptr(), size
 
     def _stage(self, spans: np.ndarray, src_index, dst_index, tokens: int, size: int) -> None:
         """Copy the step's spans and indices to the device, for the plan pass there."""
@@ -775,8 +779,9 @@ class SmallShifts:
         view = host.numpy()
         for lo, a in zip([0] + [x for x in at if x is not None], parts):
             view[lo:lo + a.nbytes] = a.reshape(-1).view(np.uint8)
-        base = self._upload(host)
-        d = self._now = self.stage_desc
+        self.staged = self._upload(host)
+        base = self.staged.data_ptr()
+        d = self.stage_desc
         d.spans, d.n_spans, d.total_tokens = base, spans.size, tokens
         for side, lo, index in ((d.src, at[0], src_index), (d.dst, at[1], dst_index)):
             side.index = None if lo is None else base + lo
@@ -798,10 +803,10 @@ class SmallShifts:
         L = _lib.lib()
         if self._last:
             d, fn = self.small_desc, L.mkv_shift_spans_small
-        elif self._now is self.desc:
+        elif self._now is self.desc and not (self._raised and error_flags is not None):
             d, fn = self.desc, L.mkv_shift_spans_planned
         else:
-            d, fn = self._now, L.mkv_shift_spans
+            d, fn = self.stage_desc, L.mkv_shift_spans
         d.error_flags = None if error_flags is None else error_flags.data_ptr()
         _lib.check(fn(ctypes.byref(d), stream))
 
