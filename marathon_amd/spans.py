@@ -617,6 +617,7 @@ class SmallShifts:
       35; 200 tokens of 12 spans 94 -> 68; 20,000 tokens of one layer 55 -> 40).
 
     Copies and launches go to the current stream; a step's device buffers are its own.
+    A graph that captured a step reads the runner's buffers: the runner outlives it.
     """
 
     def __init__(self, src: CacheSet, dst: CacheSet, *, inv_freq: torch.Tensor | None,
@@ -643,6 +644,7 @@ class SmallShifts:
         self.planned = self.staged = self.workspace = None
         self._raised = 0  # the flags of the last step's plan, made on the host
         self._keep = []
+        self._captured = []  # host buffers that captured graphs read
         with _on(self.device, self.device.index == torch.cuda.current_device()):
             static = _Staging()
             inv_off = None if inv_freq is None else static.add(self.inv_host.numpy())
@@ -737,7 +739,10 @@ class SmallShifts:
 
     def _upload(self, host: torch.Tensor) -> torch.Tensor:
         """A pinned buffer's copy on the device, in a buffer of this step's own (the
-        allocator hands it on in stream order)."""
+        allocator hands it on in stream order).  A captured copy reads ``host`` at every
+        replay, so that buffer is the runner's from then on."""
+        if torch.cuda.is_current_stream_capturing():
+            self._captured.append(host)
         buf = torch.empty(host.numel(), dtype=torch.uint8, device=self.device)
         return buf.copy_(host, non_blocking=True)
 

@@ -4,6 +4,8 @@ waits (a capture) does not count."""
 
 from __future__ import annotations
 
+import weakref
+
 import pytest
 import torch
 
@@ -106,3 +108,16 @@ def test_base_tables_live_as_long_as_launches_on_other_streams(streams):
         up.order(stream)
     assert [cs.blob.streams for cs in sets] == [{BUILD, OTHER}] * 2
     assert up.synced == {BUILD, OTHER}
+
+
+def test_a_captured_copy_keeps_its_host_buffer(streams):
+    """A graph copies from the host buffer at each replay: the runner keeps it."""
+    runner = object.__new__(spans.SmallShifts)
+    runner.device, runner._captured = torch.device("cpu"), []
+    for capturing in (False, True):
+        streams["capturing"] = capturing
+        host = torch.arange(8, dtype=torch.uint8)
+        alive = weakref.ref(host)
+        assert torch.equal(runner._upload(host), host)
+        del host
+        assert (alive() is not None) == capturing
