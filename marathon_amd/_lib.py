@@ -219,7 +219,7 @@ def lib() -> ctypes.CDLL:
 
 def binding():
     """The CPython module (``csrc/binding.cpp``), bound to the library; like :func:`lib`,
-    it raises if it has not been built."""
+    it raises if it has not been built, or was built for another library or torch."""
     global _BINDING
     if _BINDING is None:
         cdll = lib()
@@ -236,6 +236,13 @@ def binding():
                 loader = ExtensionFileLoader("marathon_binding", path)
                 module = module_from_spec(spec_from_loader("marathon_binding", loader))
                 loader.exec_module(module)
+                import torch
+
+                built = getattr(module, "abi", None), getattr(module, "torch", None)
+                if built != (MKV_ABI_VERSION, torch.__version__):
+                    raise RuntimeError(
+                        f"{path} was built for (ABI, torch) {built}, not "
+                        f"{(MKV_ABI_VERSION, torch.__version__)}; rebuild")
                 module.bind(ctypes.cast(cdll.mkv_scatter_shifted, ctypes.c_void_p).value)
                 _BINDING = module
     return _BINDING

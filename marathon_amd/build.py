@@ -111,7 +111,8 @@ def build_binding(verbose: bool = False) -> str:
     cmd = ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-ffunction-sections", "-fdata-sections", "-Wl,--gc-sections", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f"-I{INCLUDE}",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f'-DMARATHON_TORCH="{torch.__version__}"',
+           f"-I{INCLUDE}",
            "-isystem", sysconfig.get_paths()["include"],
            "-isystem", os.path.join(home, "include"),
            "-isystem", os.path.join(home, "include", "torch", "csrc", "api", "include"),

@@ -201,5 +201,12 @@ PyMODINIT_FUNC PyInit_marathon_binding() {
   s_emb_cos = PyUnicode_InternFromString("emb_cos");
   s_rotary = PyUnicode_InternFromString("rotary");
   if (!s_delta || !s_cos || !s_sgn || !s_emb_cos || !s_rotary) return nullptr;
-  return PyModule_Create(&module);
+  // what it was compiled against; the loader compares them before it calls anything
+  PyObject* m = PyModule_Create(&module);
+  if (m == nullptr || PyModule_AddIntConstant(m, "abi", MKV_ABI_VERSION) != 0 ||
+      PyModule_AddStringConstant(m, "torch", MARATHON_TORCH) != 0) {
+    Py_XDECREF(m);
+    return nullptr;
+  }
+  return m;
 }

@@ -7,6 +7,7 @@ from __future__ import annotations
 import os
 import struct
 
+import pytest
 import torch
 
 from marathon_amd import _lib
@@ -29,3 +30,18 @@ def test_binding_leaves_other_calls():
     slots = torch.zeros(2, dtype=torch.int64)
     assert scatter(src, kv, slots, 16, True, None, None, None) is None
     assert scatter(None, 3, "x", 16, True, None, None, None) is None
+
+
+@pytest.mark.parametrize("what", ["header", "torch"])
+def test_a_module_built_for_something_else_is_refused(monkeypatch, what):
+    """The module calls the library and torch by the headers it was compiled with."""
+    _lib.binding()
+    monkeypatch.setattr(_lib, "_BINDING", None)
+    if what == "header":
+        monkeypatch.setattr(_lib, "MKV_ABI_VERSION", _lib.MKV_ABI_VERSION + 1)
+    else:
+        monkeypatch.setattr(torch, "__version__", "0.0.1")
+    with pytest.raises(RuntimeError, match="rebuild"):
+        _lib.binding()
+    monkeypatch.undo()
+    assert _lib.binding().scatter is not None
