@@ -22,6 +22,7 @@ measurement or a parity check can never run anything but the HIP kernel.
 from __future__ import annotations
 
 import ctypes
+import warnings
 from dataclasses import dataclass
 
 import numpy as np
@@ -225,8 +226,18 @@ _usual_call = None  # the binding's scatter, once loaded
 
 def _load_usual_call():
     global _usual_call
-    _usual_call = _lib.binding().scatter
+    try:
+        _usual_call = _lib.binding().scatter
+    except (RuntimeError, ImportError, OSError) as e:
+        # the library alone is enough: the general path launches the same kernels
+        warnings.warn(f"scatter_shifted takes its general path, slower on the host: {e}",
+                      RuntimeWarning, stacklevel=3)
+        _usual_call = _no_usual_call
     return _usual_call
+
+
+def _no_usual_call(*args):
+    return None
 
 
 def scatter_shifted(

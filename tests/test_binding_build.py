@@ -6,11 +6,12 @@ from __future__ import annotations
 
 import os
 import struct
+import warnings
 
 import pytest
 import torch
 
-from marathon_amd import _lib
+from marathon_amd import _lib, shift_kernels
 
 PT_TLS = 7
 
@@ -45,3 +46,20 @@ def test_a_module_built_for_something_else_is_refused(monkeypatch, what):
         _lib.binding()
     monkeypatch.undo()
     assert _lib.binding().scatter is not None
+
+
+def test_scatter_shifted_does_without_the_module(monkeypatch):
+    """The general path needs only the library: with no module it takes every call, after
+    one warning."""
+    monkeypatch.setattr(shift_kernels, "_usual_call", None)
+    monkeypatch.setattr(_lib, "_BINDING", None)
+    monkeypatch.setattr(_lib, "LIB_DIR", "/nonexistent")
+    args = (torch.zeros(2, 8, 128), torch.zeros(4, 8, 16, 128), torch.zeros(2, dtype=torch.int64),
+            16, True, None)
+    with pytest.warns(RuntimeWarning, match="marathon_binding.so"):
+        with pytest.raises(RuntimeError, match="not on a HIP device"):
+            shift_kernels.scatter_shifted(*args)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        with pytest.raises(RuntimeError, match="not on a HIP device"):
+            shift_kernels.scatter_shifted(*args)
