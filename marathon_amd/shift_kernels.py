@@ -11,7 +11,7 @@ Same names, argument meanings and error behaviour as the reference module:
   (shift_kernels.py:166-210).  One call is one HIP launch on the current stream.
 * :func:`use_hip` -- the analogue of ``use_triton`` (shift_kernels.py:162-163).
 * :func:`warmup` -- kept for the connector's call (vllm_shift_connector.py:404-405);
-  the kernels are compiled ahead of time, so it only loads the library.
+  the kernels are compiled ahead of time, so it only loads the library and the module.
 
 Divergence, on purpose: there is no torch fallback.  The reference's
 ``scatter_shifted`` falls back to ``scatter_shifted_torch`` off-GPU
@@ -342,10 +342,13 @@ def scatter_shifted(
 
 
 def warmup(kv: torch.Tensor, block_size: int, hnd: bool) -> None:
-    """Load the library before the first real load (shift_kernels.py:213-238).
+    """Load the library and the CPython module before the first real load
+    (shift_kernels.py:213-238).
 
     The reference pre-compiles its Triton specialisations here; HIP kernels are
-    compiled ahead of time, so there is nothing to compile -- only the library load.
+    compiled ahead of time, so there is nothing to compile -- only the two to load.
     """
     if use_hip(kv):
         _lib.lib()
+        if _usual_call is None:
+            _load_usual_call()

@@ -7,6 +7,7 @@ from __future__ import annotations
 import os
 import struct
 import warnings
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -63,3 +64,11 @@ def test_scatter_shifted_does_without_the_module(monkeypatch):
         warnings.simplefilter("error")
         with pytest.raises(RuntimeError, match="not on a HIP device"):
             shift_kernels.scatter_shifted(*args)
+
+
+def test_warmup_loads_what_the_first_call_needs(monkeypatch):
+    monkeypatch.setattr(shift_kernels, "_usual_call", None)
+    shift_kernels.warmup(SimpleNamespace(is_cuda=False), 16, True)
+    assert shift_kernels._usual_call is None
+    shift_kernels.warmup(SimpleNamespace(is_cuda=True), 16, True)
+    assert shift_kernels._usual_call is _lib.binding().scatter
