@@ -845,7 +845,7 @@ class ShiftSaver:
         """Flush the deferred layers: one launch per distinct list of saves (a step has
         one).  Returns the token-layers saved; 0 when nothing is pending."""
         pending = self._pending[:]
-        self._pending.clear()
+        del self._pending[:len(pending)]  # not what another thread has recorded since
         if not pending:
             return 0
         saves = pending[0][2]

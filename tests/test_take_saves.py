@@ -76,3 +76,23 @@ def test_deferred_layers_are_grouped_by_their_saves():
     saver.save_kv_layer("e", "E", two)
     assert saver.wait_for_save() == 1 and seen[2] == (["e"], ["E"], two)
     assert saver.wait_for_save() == 0
+
+
+def test_a_layer_recorded_while_the_step_is_flushed_is_kept():
+    """A hook on another thread between the flush's copy and its clearing of the list."""
+    saver = ShiftSaver(BlockShiftStore(64, "cpu"), 16, deferred=True)
+    one, two, seen = [1], [1], []
+
+    class Pending(list):
+        def __getitem__(self, key):
+            got = super().__getitem__(key)
+            if self:
+                self.append(("late", "LATE", two))
+            return got
+
+    saver._pending = Pending([("a", "A", one)])
+    saver._plan = lambda names, caches, saves: seen.append((list(names), saves)) or 1
+    assert saver.wait_for_save() == 1
+    saver._pending = list(saver._pending)
+    assert saver.wait_for_save() == 1
+    assert seen == [(["a"], one), (["late"], two)] and seen[1][1] is two
