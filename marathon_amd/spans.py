@@ -816,6 +816,12 @@ class SmallShifts:
         _lib.check(fn(ctypes.byref(d), stream))
 
     @property
+    def direct(self) -> bool:
+        """Whether the last step runs as one launch, with no plan pass (as
+        :attr:`ShiftPlan.direct`, for a connector's ``last_plan``)."""
+        return bool(self._last) or self._now is self.desc
+
+    @property
     def algorithmic_bytes(self) -> int:
         eb = self.dst.first.element_size()
         return 2 * self.tokens * self.dst.layers * self.dst.heads * 2 * self.dst.head_size * eb

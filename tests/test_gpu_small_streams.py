@@ -41,6 +41,7 @@ def test_steps_wait_for_uploads_on_another_stream(gpu, form, tokens, dtype):
     got = {"launch": bool(one._last), "planned": not one._last and one._now is one.desc,
            "staged": one._now is one.stage_desc}
     assert [k for k, v in got.items() if v] == [form]
+    assert one.direct == (form != "staged")
     want = [bits(t) for t in out]
     assert any(w.any() for w in want)
     for t in out:
