@@ -23,6 +23,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import struct
+import threading
 from dataclasses import dataclass
 from itertools import chain
 
@@ -645,6 +646,7 @@ class SmallShifts:
         self._raised = 0  # the flags of the last step's plan, made on the host
         self._keep = []
         self._captured = []  # host buffers that captured graphs read
+        self._lock = threading.RLock()
         with _on(self.device, self.device.index == torch.cuda.current_device()):
             static = _Staging()
             inv_off = None if inv_freq is None else static.add(self.inv_host.numpy())
@@ -697,6 +699,10 @@ class SmallShifts:
         Up to ``MKV_SMALL_MAX_SPANS`` spans and ``MKV_SMALL_MAX_INDEX`` index entries a
         side, the rows and windows travel in the launch itself
         (``mkv_shift_spans_small``)."""
+        with self._lock:  # a runner's threads share its descriptors
+            self._run(rows, src_index, dst_index, error_flags, tokens)
+
+    def _run(self, rows: list, src_index, dst_index, error_flags, tokens) -> None:
         n = len(rows)
         n_src = 0 if src_index is None else src_index.size
         n_dst = 0 if dst_index is None else dst_index.size
@@ -803,17 +809,18 @@ class SmallShifts:
         if stream is None:
             stream = current_stream(self.device)
         stream = int(stream)
-        if stream not in self._uploads.synced:
-            self._uploads.order(stream)
         L = _lib.lib()
-        if self._last:
-            d, fn = self.small_desc, L.mkv_shift_spans_small
-        elif self._now is self.desc and not (self._raised and error_flags is not None):
-            d, fn = self.desc, L.mkv_shift_spans_planned
-        else:
-            d, fn = self.stage_desc, L.mkv_shift_spans
-        d.error_flags = None if error_flags is None else error_flags.data_ptr()
-        _lib.check(fn(ctypes.byref(d), stream))
+        with self._lock:
+            if stream not in self._uploads.synced:
+                self._uploads.order(stream)
+            if self._last:
+                d, fn = self.small_desc, L.mkv_shift_spans_small
+            elif self._now is self.desc and not (self._raised and error_flags is not None):
+                d, fn = self.desc, L.mkv_shift_spans_planned
+            else:
+                d, fn = self.stage_desc, L.mkv_shift_spans
+            d.error_flags = None if error_flags is None else error_flags.data_ptr()
+            _lib.check(fn(ctypes.byref(d), stream))
 
     @property
     def direct(self) -> bool:
