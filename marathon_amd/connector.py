@@ -206,11 +206,6 @@ def _host(index) -> np.ndarray | None:
     return index.numpy()
 
 
-def _on_device(index) -> bool:
-    """Whether a step's index is on the GPU: a plan reads it there, in place."""
-    return isinstance(index, torch.Tensor) and index.is_cuda
-
-
 def _int32_table(t) -> np.ndarray:
     if isinstance(t, np.ndarray) and t.dtype == np.int32:
         return t.reshape(-1)
@@ -449,7 +444,8 @@ class ShiftLoader:
         if self.timing:
             torch.cuda.synchronize(dst.first.device)
             t0 = time.perf_counter()
-        small = None if _on_device(dst_index) else self._small.get(
+        # (slots on the GPU: a plan reads them there, in place)
+        small = None if dst_mode == "slots" and dst_index.is_cuda else self._small.get(
             src, dst, src_mode, dst_mode, self.inv_freq, k_scale)
         if small is not None and small.fits(len(rows), tokens):  # no plan to build
             small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)
@@ -807,7 +803,8 @@ class ShiftSaver:
     def _launch(self, names: list, paged, dst, rows: list, src_mode, src_index, dst_mode,
                 dst_index) -> int:
         tokens = sum([r[4] for r in rows])
-        small = None if _on_device(src_index) else self._small.get(
+        # (slots on the GPU: a plan reads them there, in place)
+        small = None if src_mode == "slots" and src_index.is_cuda else self._small.get(
             paged, dst, src_mode, dst_mode, None)
         if small is not None and small.fits(len(rows), tokens):  # no plan to build
             small.run(rows, _host(src_index), _host(dst_index), tokens=tokens)

@@ -646,7 +646,7 @@ class SmallShifts:
         self._raised = 0  # the flags of the last step's plan, made on the host
         self._keep = []
         self._captured = []  # host buffers that captured graphs read
-        self._lock = threading.RLock()
+        self._lock = threading.Lock()
         with _on(self.device, self.device.index == torch.cuda.current_device()):
             static = _Staging()
             inv_off = None if inv_freq is None else static.add(self.inv_host.numpy())
@@ -703,6 +703,7 @@ class SmallShifts:
             self._run(rows, src_index, dst_index, error_flags, tokens)
 
     def _run(self, rows: list, src_index, dst_index, error_flags, tokens) -> None:
+        stream = current_stream(self.device)
         n = len(rows)
         n_src = 0 if src_index is None else src_index.size
         n_dst = 0 if dst_index is None else dst_index.size
@@ -727,7 +728,7 @@ class SmallShifts:
             d.dst.index = self._h_addr[2] if n_dst else None
             d.dst.index_len = n_dst
             self._last = (True,)  # a relaunch reads the host buffers again
-            self.launch(error_flags=error_flags)
+            self._enqueue(stream, error_flags)
             return
         self._last = ()
         self.tokens = tokens
@@ -737,23 +738,23 @@ class SmallShifts:
         _span_struct(n).pack_into(spans.view(np.uint8), 0, *chain.from_iterable(rows))
         self._raised = 0
         if size <= HOST_PLAN_MAX_BYTES:
-            self._plan_here(spans, src_index, dst_index, tokens, size)
+            self._plan_here(spans, src_index, dst_index, tokens, size, stream)
         if size > HOST_PLAN_MAX_BYTES or self._raised:
-            self._stage(spans, src_index, dst_index, tokens, size)
+            self._stage(spans, src_index, dst_index, tokens, size, stream)
         self._now = self.desc if size <= HOST_PLAN_MAX_BYTES else self.stage_desc
-        self.launch(error_flags=error_flags)
+        self._enqueue(stream, error_flags)
 
-    def _upload(self, host: torch.Tensor) -> torch.Tensor:
+    def _upload(self, host: torch.Tensor, stream: int) -> torch.Tensor:
         """A pinned buffer's copy on the device, in a buffer of this step's own (the
         allocator hands it on in stream order).  A captured copy reads ``host`` at every
         replay, so that buffer is the runner's from then on."""
-        if torch.cuda.is_current_stream_capturing():
+        if stream and torch.cuda.is_current_stream_capturing():  # (stream 0 never is)
             self._captured.append(host)
         buf = torch.empty(host.numel(), dtype=torch.uint8, device=self.device)
         return buf.copy_(host, non_blocking=True)
 
     def _plan_here(self, spans: np.ndarray, src_index, dst_index, tokens: int,
-                   size: int) -> None:
+                   size: int, stream: int) -> None:
         """Plan the step on the host.  The plan holds no rows that cannot be moved, so it
         raises no flags when launched: such a step is staged as well, for launches that
         ask for them."""
@@ -772,12 +773,13 @@ class SmallShifts:
         h.workspace, h.workspace_bytes = host.data_ptr(), size
         _lib.check(_lib.lib().mkv_plan_host(ctypes.byref(h), self._flags_at))
         self._raised = int(self._flags[0])
-        self.planned = self._upload(host)
+        self.planned = self._upload(host, stream)
         d = self.desc
         d.n_spans, d.total_tokens = spans.size, tokens
         d.workspace, d.workspace_bytes = self.planned.data_ptr(), size
 
-    def _stage(self, spans: np.ndarray, src_index, dst_index, tokens: int, size: int) -> None:
+    def _stage(self, spans: np.ndarray, src_index, dst_index, tokens: int, size: int,
+               stream: int) -> None:
         """Copy the step's spans and indices to the device, for the plan pass there."""
         parts, end = [spans], spans.nbytes
         at = [None, None]
@@ -790,7 +792,7 @@ class SmallShifts:
         view = host.numpy()
         for lo, a in zip([0] + [x for x in at if x is not None], parts):
             view[lo:lo + a.nbytes] = a.reshape(-1).view(np.uint8)
-        self.staged = self._upload(host)
+        self.staged = self._upload(host, stream)
         base = self.staged.data_ptr()
         d = self.stage_desc
         d.spans, d.n_spans, d.total_tokens = base, spans.size, tokens
@@ -803,24 +805,26 @@ class SmallShifts:
     def launch(self, stream: int | None = None, error_flags: torch.Tensor | None = None) -> None:
         """(Re)launch the last step on ``stream`` (default: current); a step that copied
         anything to the device must run on the stream it was copied on."""
-        if self.device.index != torch.cuda.current_device():
-            with torch.cuda.device(self.device):  # launches go to the current device
-                return self.launch(stream, error_flags)
         if stream is None:
             stream = current_stream(self.device)
-        stream = int(stream)
-        L = _lib.lib()
         with self._lock:
-            if stream not in self._uploads.synced:
-                self._uploads.order(stream)
-            if self._last:
-                d, fn = self.small_desc, L.mkv_shift_spans_small
-            elif self._now is self.desc and not (self._raised and error_flags is not None):
-                d, fn = self.desc, L.mkv_shift_spans_planned
-            else:
-                d, fn = self.stage_desc, L.mkv_shift_spans
-            d.error_flags = None if error_flags is None else error_flags.data_ptr()
-            _lib.check(fn(ctypes.byref(d), stream))
+            self._enqueue(int(stream), error_flags)
+
+    def _enqueue(self, stream: int, error_flags) -> None:
+        if self.device.index != torch.cuda.current_device():
+            with torch.cuda.device(self.device):  # launches go to the current device
+                return self._enqueue(stream, error_flags)
+        if stream not in self._uploads.synced:
+            self._uploads.order(stream)
+        L = _lib.lib()
+        if self._last:
+            d, fn = self.small_desc, L.mkv_shift_spans_small
+        elif self._now is self.desc and not (self._raised and error_flags is not None):
+            d, fn = self.desc, L.mkv_shift_spans_planned
+        else:
+            d, fn = self.stage_desc, L.mkv_shift_spans
+        d.error_flags = None if error_flags is None else error_flags.data_ptr()
+        _lib.check(fn(ctypes.byref(d), stream))
 
     @property
     def direct(self) -> bool:

@@ -49,15 +49,14 @@ def test_a_launch_is_of_its_own_thread_s_step(monkeypatch, form):
     def step(n):
         runner.run([(0, 0, 0, 0, n, 0, 0, 0)], index, None)
 
-    def stream_asked_for(device):
+    def device_asked_for():
         if not busy.is_set():  # this thread's step has its descriptor and not its launch yet
             busy.set()
             other.start()
             other.join(0.3)
-        return 0x10
 
     other = threading.Thread(target=step, args=(theirs,))
-    monkeypatch.setattr(spans, "current_stream", stream_asked_for)
+    monkeypatch.setattr(torch.cuda, "current_device", device_asked_for)
     step(mine)
     other.join()
     fn = {"launch": "mkv_shift_spans_small", "planned": "mkv_shift_spans_planned",

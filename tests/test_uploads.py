@@ -118,6 +118,6 @@ def test_a_captured_copy_keeps_its_host_buffer(streams):
         streams["capturing"] = capturing
         host = torch.arange(8, dtype=torch.uint8)
         alive = weakref.ref(host)
-        assert torch.equal(runner._upload(host), host)
+        assert torch.equal(runner._upload(host, OTHER), host)
         del host
         assert (alive() is not None) == capturing
