@@ -5,7 +5,8 @@
 // interface, checks what that function checks and calls mkv_scatter_shifted on the current
 // stream.  Through Python methods and ctypes the same call spent 3.6 us of its 6.7 around
 // the launch, longer than the kernel of a short span runs (2.4 us for 300 tokens), so a loop
-// over layers was bound by it: 28 calls of 301 fp16 tokens 165 -> 87 us.
+// over layers was bound by it: 28 calls of 301 fp16 tokens 165 -> 79 to 108 us, a process
+// settling at one figure or another between these (2.8 to 3.8 us a call).
 //
 // Returns the library's status, or None wherever the call is not the usual one (tensors
 // that need a copy or a conversion, subclasses and wrapped tensors, another current device,

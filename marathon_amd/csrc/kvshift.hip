@@ -208,7 +208,8 @@ static_assert(MKV_XCDS >= 1, "MKV_XCDS");
 #ifndef MKV_LAYER_MAJOR_MIN_TOKENS
 #define MKV_LAYER_MAJOR_MIN_TOKENS 100000
 #endif
-// Which rows a wave's passes take when it makes more than one (fp8, fp32): 0 = pass u of
+// Which rows a wave's passes take when it makes more than one (fp8; a one-layer launch of
+// two or four, any type): 0 = pass u of
 // wave w takes the tile's row group w + waves * u (the waves interleave); 1 = w * passes + u
 // (a wave's passes take adjacent row groups: for 8 heads, adjacent tokens).
 #ifndef MKV_PASS_MAJOR
@@ -1943,19 +1944,22 @@ int launch_any(int dtype, bool uniform, int direct_layers, const ShiftParams& sp
 
 // Passes a wave of a one-layer launch makes, by the waves the launch would have at one pass
 // each (`waves`, of 2 KB read and 2 KB written).  A launch this small is over in one or two
-// generations of resident waves, so its shape matters more than its inner loop: the fewest
-// passes that let every wave be resident at once with at most four waves on a SIMD (256
-// CUs of 4 SIMDs, and every variant's registers allow four; fp8's per-lane one, three).
-// Past that a launch takes several generations either way, and one pass overlaps loads and
-// stores best.  Measured, 40 launches back to back, us a launch at 1 / 2 / 4 passes (8
-// heads of 128; 256-thread workgroups, a few percent ahead of 128 wherever the passes
-// differ):
-//   bf16   8 MB (1,952 waves) 4.53 / 4.61 / 5.71   16 MB (3,906) 5.30 / 5.39 / 6.01
-//         33 MB (8,056) 7.67 / 7.12 / 7.71         50 MB (12,206) 10.63 / 9.65 / 9.70
-//         67 MB (16,356) 13.2 / 14.6 / 13.9        200 MB 34.1 / 36.7 / 39.6
-//   fp32  33 MB 7.54 / 7.23 / 7.62   50 MB 10.2 / 10.5 / 9.95   67 MB 12.7 / 13.9 / 12.8
-//   fp8   16 MB 6.87 / 6.22 / 7.40   50 MB 12.8 / 13.7 / 11.3   67 MB 15.7 / 16.3 / 13.9
-//   bf16, 2 heads: 42 MB 10.0 / 10.0 / 8.5, 50 MB 11.3 / 11.1 / 9.1, 67 MB 14.1 / 14.5 / 14.6
+// generations of resident waves, so its shape matters more than its inner loop: with two
+// passes, then four, its waves are all resident at once for longer, and past that a launch
+// takes several generations either way and one pass (fp8 two) overlaps loads and stores
+// best.  The lines are set by these times, in waves a SIMD (256 CUs of 4 SIMDs), one for all
+// types and head counts where they differ little.  Launches back to back, us each at 1 / 2 /
+// 4 passes (256-thread workgroups, a few percent ahead of 128 wherever the passes differ):
+//   bf16, 8 heads of 128, by waves: 1,952 3.2 / 4.0 / 5.1   3,072 4.5 / 4.6 / 5.3
+//     4,096 4.9 / 5.0 / 5.6   6,144 6.8 / 6.2 / 6.6   8,192 7.8 / 7.2 / 7.4
+//     10,240 9.4 / 8.2 / 8.8   12,288 10.6 / 9.6 / 9.5   14,336 12.2 / 13.4 / 12.5
+//     16,356 13.1 / 14.7 / 13.5   (200 MB) 34.1 / 36.7 / 39.6
+//   bf16, 2 heads: 10,240 10.0 / 10.0 / 8.5   12,206 11.3 / 11.1 / 9.1
+//     16,356 14.1 / 14.5 / 14.6
+//   fp32: 4,096 4.7 / 4.6 / 6.1   8,192 7.5 / 7.0 / 7.6   12,288 10.2 / 10.5 / 10.0
+//     16,356 12.7 / 13.9 / 12.8
+//   fp8: 3,072 5.7 / 5.6 / 7.0   4,096 6.5 / 5.9 / 7.3   8,192 9.8 / 8.5 / 9.4
+//     12,288 12.7 / 13.6 / 11.2   16,384 15.6 / 16.1 / 14.0
 constexpr int64_t kSimds = 1024;
 
 int scatter_passes(int dtype, const Geometry& g, int64_t tokens, int heads) {

@@ -38,32 +38,38 @@ MODES = {"flat": _lib.MKV_ADDR_FLAT, "slots": _lib.MKV_ADDR_SLOTS, "table": _lib
 #: Shifts of at most this many (token, layer) rows take the library's direct path when
 #: eligible: one launch instead of the plan pass plus the shift.  Measured on MI355X
 #: (bf16, 8 heads, 40 layers, one span, flat store -> HND cache through shuffled slots;
-#: bench.py's plan_variants): 16, 64, 256 and 512 tokens run in 6.6, 8.8, 21.8 and
-#: 34.3 us direct against 10.2, 11.9, 22.5 and 36.8 us; from 1,024 tokens the two-launch
-#: path is faster (61.6 against 63.5 us): a direct workgroup resolves its token (span,
-#: then slot) before it can load its data, where a record from the plan pass carries the
-#: token's rows.  Above 2,560 rows the direct kernel moves four layers per workgroup.
+#: bench.py's plan_variants): 16, 64, 256 and 512 tokens run in 6.6, 9.4, 19.7 and
+#: 33.9 us direct against 9.2, 11.8, 20.9 and 34.9 us.  Launched back to back (2 spans) the
+#: two are within 2% of each other from 300 to 700 tokens (300 19.9 / 19.7, 511 31.7 /
+#: 31.5), and at 1,024 the two launches are ahead (62.2 / 57.6): a direct workgroup resolves
+#: its token (span, then slot) before it can load its data, where a record from the plan
+#: pass carries the token's rows.  Above 2,560 rows the direct kernel moves four layers per
+#: workgroup.
 DIRECT_MAX_TOKEN_LAYERS = 20480
 #: The most bytes of K and V such a shift may read, by element size (default the last):
 #: resolving a token again for each of its layers costs a direct workgroup the more, the
 #: more workgroups a token and layer take and the fewer bytes each moves.  Kept plans of 2
-#: spans x 40 layers, us a launch, direct / two launches: fp8 8 heads of 128, 150 tokens (12
-#: MB) 9.9 / 11.2, 200 (16 MB) 13.0 / 12.1, 511 24.8 / 21.1; 16 heads, 64 tokens (10 MB) 9.4
-#: / 10.7, 100 (16 MB) 14.1 / 12.2, 511 46.2 / 37.2; bf16 16 heads, 303 tokens (99 MB) 37.7
-#: / 39.6, 400 (131 MB) 50.6 / 49.2, 511 64.9 / 59.9; fp32 8 heads, 511 tokens (167 MB) 61.9
-#: / 58.7.
+#: spans x 40 layers, us a launch, direct / two launches: fp8 8 heads of 128, 100 tokens (8
+#: MB) 9.6 / 9.8, 150 (12 MB) 11.0 / 10.8, 200 (16 MB) 13.8 / 11.7, 511 25.0 / 19.9; 16
+#: heads, 64 tokens (10 MB) 9.8 / 9.8, 100 (16 MB) 14.4 / 12.6, 511 45.7 / 32.3; bf16 16
+#: heads, 303 tokens (95 MB) 36.4 / 37.0, 400 (125 MB) 47.6 / 46.5, 511 61.7 / 58.2.  fp32
+#: shares bf16's line and ties well below it: 8 heads, 100 tokens (31 MB) 14.9 / 14.8, 200
+#: (62 MB) 25.7 / 23.8, 300 (94 MB) 37.4 / 35.5, 511 61.7 / 57.3.
 DIRECT_MAX_BYTES = {1: 14 << 20, None: 120 << 20}
 #: SmallShifts puts a step's spans and index windows in the launch's own arguments up to
-#: this many (token, layer) rows: that saves the host its staging copy, but every
-#: workgroup then reads the arguments, which costs more than the copy from about 64
-#: tokens x 40 layers on (12.6 against 9.6 us of GPU time; 34 against 22 at 256).
+#: this many (token, layer) rows: that saves the host its copy, but every workgroup then
+#: reads the arguments and resolves its token.  Whole calls back to back, 40 layers bf16, us,
+#: in the launch / planned on the host: 16 tokens 6.5 / 15.4, 64 8.6 / 15.5, 96 11.5 /
+#: 15.8, 128 15.6 / 16.5, 256 25.0 / 20.0.  The line, 64 tokens, is where the GPU's own time
+#: crosses (8.5 us against a copy's 2.3 and a record kernel's 6.0): beyond it the step in the
+#: launch is bound by the GPU, the planned one by the host.
 SMALL_ARGS_MAX_TOKEN_LAYERS = 2560
 #: SmallShifts plans a step on the host where its plan is at most this many bytes: a host
 #: copy of up to 16 KB is a small kernel on the stream (2.3 us), a larger one goes through a
-#: copy engine that the stream waits for, longer than for the 5.4 us plan pass it replaces.
-#: Loads of 36 layers, calls back to back, us, plan pass / host plan: bf16 303 tokens 51 /
-#: 31, 400 tokens 50 / 31, fp8 54 / 34; past 16 KB bf16 600 tokens 44 / 53, 800 tokens 53 /
-#: 62, fp8 37 / 43, 1,500 tokens 53 / 63.
+#: copy engine that the stream waits for, longer than for the 4 us plan pass it replaces.
+#: Loads of 36 layers, calls back to back, us, plan pass / host plan: bf16 303 tokens 29.7 /
+#: 26.6, 400 31.6 / 26.9, 480 (16 KB) 34.7 / 30.5, fp8 400 31.4 / 28.4; past 16 KB bf16 600
+#: tokens 41 / 52, 800 50 / 61, fp8 600 33 / 40, 1,500 53 / 64.
 HOST_PLAN_MAX_BYTES = 16384
 
 
@@ -342,6 +348,11 @@ class ShiftPlan:
     22,141 tokens when the plan is built; a caller that builds a plan for a single launch
     with the host on its critical path (the connector's per-step loads) passes
     ``"none"``.
+
+    A plan that is not direct owns its workspace, which each launch fills again.  Launches of
+    one plan on several streams write the same bytes there, so they need no order between
+    them, except with more spans than one descriptor takes (``MKV_MAX_SPANS``) or an order
+    sorted on the device: those launches must follow one another.
     """
 
     def __init__(
@@ -614,8 +625,8 @@ class SmallShifts:
     * as a plan made here (``mkv_plan_host``), copied to the device and launched alone
       (``mkv_shift_spans_planned``), where the plan fits :data:`HOST_PLAN_MAX_BYTES`;
     * as they are, in one pinned copy, for the plan pass and the shift (whole calls against
-      the direct path and its tables: 511 tokens x 40 layers, bf16 51 -> 41 us, fp8 54 ->
-      35; 200 tokens of 12 spans 94 -> 68; 20,000 tokens of one layer 55 -> 40).
+      the direct path and its tables: 511 tokens x 40 layers, bf16 51 -> 38.5 us, fp8 54 ->
+      29.4; 200 tokens of 12 spans 94 -> 60.5; 20,000 tokens of one layer 55 -> 40).
 
     Copies and launches go to the current stream; a step's device buffers are its own.
     A graph that captured a step reads the runner's buffers: the runner outlives it.

@@ -2,8 +2,8 @@
 
 Up to 8 spans and 64 index entries a side, a step travels in the launch's own kernel
 arguments (``mkv_shift_spans_small``: rows and index windows from host memory, rotation
-tables computed in the kernel); larger direct steps go through the runner's device
-buffer (``mkv_shift_spans`` direct path).  Seeded random steps over element types,
+tables computed in the kernel); larger steps are planned on the host and copied to the
+device (``mkv_shift_spans_planned``).  Seeded random steps over element types,
 source and destination modes, groups and deltas of every magnitude, run one after
 another through one runner, each checked byte for byte against the oracle.
 """
