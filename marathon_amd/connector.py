@@ -92,7 +92,7 @@ class Save:
     """
 
     session: str
-    slots: torch.Tensor | None  # int64 [T]
+    slots: torch.Tensor | None  # int64 [T], on the host or the GPU
     dst_start: int
     block_ids: object = None  # the request's block table (device-side slots)
     n_tokens: int = 0
@@ -119,7 +119,8 @@ class Load:
     """
 
     session: str
-    slots: torch.Tensor | None  # int64 [T]: destination slots of positions [lo, hi)
+    slots: torch.Tensor | None  # int64 [T]: destination slots of positions [lo, hi), on
+    # the host or the GPU
     src_start: int  # first source position in the session's store
     delta: int
     block_ids: object = None  # the request's block table (device-side slots)
@@ -729,8 +730,8 @@ class ShiftSaver:
         self._small = _SmallRunners()
 
     def _geometry(self, caches: list) -> tuple:
-        """``(row_shape, dtype, device, paged CacheSet)`` of a step's paged caches, worked
-        out once per distinct tuple of cache tensors (vLLM passes the same ones every
+        """``(row_shape, dtype, device, paged CacheSet, caches)`` of a step's paged caches,
+        worked out once per distinct tuple of cache tensors (vLLM passes the same ones every
         step)."""
         # keyed by the tensors' ids (a tuple of tensors would hash each tensor through
         # Python); the entry holds the tensors, so no id is reused meanwhile (its CacheSet
@@ -749,10 +750,10 @@ class ShiftSaver:
             if len(self._geo) >= 64:  # caches replaced many times over
                 self._geo.clear()
             hit = self._geo[key] = (row_shape, first.dtype, first.device, paged, tuple(caches))
-        return hit[:4]
+        return hit
 
     def _plan(self, names: list, caches: list, saves: list) -> int:
-        row_shape, dtype, device, paged = self._geometry(caches)
+        row_shape, dtype, device, paged, _ = self._geometry(caches)
         if isinstance(self.store, BlockShiftStore):
             return self._plan_blocks(names, saves, row_shape, dtype, device, paged)
         groups: dict[str, int] = {}

@@ -673,6 +673,7 @@ class SmallShifts:
             self._keep.append(blob)
             sides = [cs.device_tables(self.device)[:3] for cs in (src, dst)]
             self._uploads = _Uploads(self.device, (src, dst), self._keep)
+            self._synced = self._uploads.synced
         base = blob.data_ptr()
         d = self.desc = _lib.ShiftDesc()
         d.inv_freq = None if inv_off is None else base + inv_off
@@ -711,49 +712,46 @@ class SmallShifts:
         side, the rows and windows travel in the launch itself
         (``mkv_shift_spans_small``)."""
         with self._lock:  # a runner's threads share its descriptors
-            self._run(rows, src_index, dst_index, error_flags, tokens)
-
-    def _run(self, rows: list, src_index, dst_index, error_flags, tokens) -> None:
-        stream = current_stream(self.device)
-        n = len(rows)
-        n_src = 0 if src_index is None else src_index.size
-        n_dst = 0 if dst_index is None else dst_index.size
-        if tokens is None:
-            tokens = sum(max(int(r[4]), 0) for r in rows)
-        if (self.eligible_geometry and n <= _lib.MKV_SMALL_MAX_SPANS
-                and n_src <= _lib.MKV_SMALL_MAX_INDEX and n_dst <= _lib.MKV_SMALL_MAX_INDEX
-                and tokens * self.dst.layers <= SMALL_ARGS_MAX_TOKEN_LAYERS):
-            hs = self._h_spans
-            for i, r in enumerate(rows):
-                hs[i] = r
-            if n_src:
-                self._h_index[0][:n_src] = src_index
-            if n_dst:
-                self._h_index[1][:n_dst] = dst_index
-            d = self.small_desc
-            d.spans = self._h_addr[0]
-            d.n_spans = n
-            d.total_tokens = self.tokens = tokens
-            d.src.index = self._h_addr[1] if n_src else None
-            d.src.index_len = n_src
-            d.dst.index = self._h_addr[2] if n_dst else None
-            d.dst.index_len = n_dst
-            self._last = (True,)  # a relaunch reads the host buffers again
+            stream = current_stream(self.device)
+            n = len(rows)
+            n_src = 0 if src_index is None else src_index.size
+            n_dst = 0 if dst_index is None else dst_index.size
+            if tokens is None:
+                tokens = sum(max(int(r[4]), 0) for r in rows)
+            if (self.eligible_geometry and n <= _lib.MKV_SMALL_MAX_SPANS
+                    and n_src <= _lib.MKV_SMALL_MAX_INDEX and n_dst <= _lib.MKV_SMALL_MAX_INDEX
+                    and tokens * self.dst.layers <= SMALL_ARGS_MAX_TOKEN_LAYERS):
+                hs = self._h_spans
+                for i, r in enumerate(rows):
+                    hs[i] = r
+                if n_src:
+                    self._h_index[0][:n_src] = src_index
+                if n_dst:
+                    self._h_index[1][:n_dst] = dst_index
+                d = self.small_desc
+                d.spans = self._h_addr[0]
+                d.n_spans = n
+                d.total_tokens = self.tokens = tokens
+                d.src.index = self._h_addr[1] if n_src else None
+                d.src.index_len = n_src
+                d.dst.index = self._h_addr[2] if n_dst else None
+                d.dst.index_len = n_dst
+                self._last = (True,)  # a relaunch reads the host buffers again
+                self._enqueue(stream, error_flags)
+                return
+            self._last = ()
+            self.tokens = tokens
+            # mkv_shift_workspace_size: the spans' tables, then 32 bytes a token
+            size = (n * 8 * self.rotary + 255) // 256 * 256 + 32 * tokens
+            spans = np.empty(n, dtype=_lib.SPAN_DTYPE)
+            _span_struct(n).pack_into(spans.view(np.uint8), 0, *chain.from_iterable(rows))
+            self._raised = 0
+            if size <= HOST_PLAN_MAX_BYTES:
+                self._plan_here(spans, src_index, dst_index, tokens, size, stream)
+            if size > HOST_PLAN_MAX_BYTES or self._raised:
+                self._stage(spans, src_index, dst_index, tokens, size, stream)
+            self._now = self.desc if size <= HOST_PLAN_MAX_BYTES else self.stage_desc
             self._enqueue(stream, error_flags)
-            return
-        self._last = ()
-        self.tokens = tokens
-        # mkv_shift_workspace_size: the spans' tables, then 32 bytes a token
-        size = (n * 8 * self.rotary + 255) // 256 * 256 + 32 * tokens
-        spans = np.empty(n, dtype=_lib.SPAN_DTYPE)
-        _span_struct(n).pack_into(spans.view(np.uint8), 0, *chain.from_iterable(rows))
-        self._raised = 0
-        if size <= HOST_PLAN_MAX_BYTES:
-            self._plan_here(spans, src_index, dst_index, tokens, size, stream)
-        if size > HOST_PLAN_MAX_BYTES or self._raised:
-            self._stage(spans, src_index, dst_index, tokens, size, stream)
-        self._now = self.desc if size <= HOST_PLAN_MAX_BYTES else self.stage_desc
-        self._enqueue(stream, error_flags)
 
     def _upload(self, host: torch.Tensor, stream: int) -> torch.Tensor:
         """A pinned buffer's copy on the device, in a buffer of this step's own (the
@@ -825,7 +823,7 @@ class SmallShifts:
         if self.device.index != torch.cuda.current_device():
             with torch.cuda.device(self.device):  # launches go to the current device
                 return self._enqueue(stream, error_flags)
-        if stream not in self._uploads.synced:
+        if stream not in self._synced:
             self._uploads.order(stream)
         L = _lib.lib()
         if self._last:
